@@ -368,11 +368,17 @@ __device__ __forceinline__ void mixed_cg_after_iteration(VolState<A>* s, A rz) {
         s->status = ST_UPDATE;
         return;
     }
+    if (s->mg && ++s->mg_since >= s->mg_stall) {
+        s->mg = 0;
+        s->status = ST_FRESH;
+        return;
+    }
+    s->first = 0;
+    s->status = ST_RUNNING;
+    if (s->mg) return;   // r.z and beta come from the next multigrid cycle
     const A absold = s->absnew;
     s->absnew = rz;
     s->beta = s->absnew / absold;
-    s->first = 0;
-    s->status = ST_RUNNING;
 }
 
 // Scalar update of one volume after a pass, from the pass's dot products `tot` (run by one
@@ -487,6 +493,7 @@ __device__ void mixres_update(VolState<double>* s, const double* tot) {
     }
     s->refinements += 1;
     s->discard = 0;
+    s->mg_since = 0;
     s->r64sq = tot[0];
     if (s->b64sq == 0.0 || !(s->r64sq > s->otol * s->otol * s->b64sq) || s->iter >= s->maxiter) {
         s->status = ST_IDLE;
@@ -501,6 +508,8 @@ __device__ void mixres_update(VolState<double>* s, const double* tot) {
             if (s->refinements > 1) s->restarts += 1;
             s->first = 1;
             s->absnew = tot[3];
+        } else if (s->mg) {   // r.z and beta come from the next multigrid cycle
+            s->first = 0;
         } else {
             const double absold = s->absnew;
             s->absnew = tot[3];
@@ -533,6 +542,31 @@ __device__ void mixres_update(VolState<double>* s, const double* tot) {
     s->rho = rho_new;
     s->beta = (s->rho / s->rho_old) * (s->alpha / s->omega);
     s->status = ST_RUNNING;
+}
+
+// Element of slot k of row (y, z) in the padded per-colour layout (a ghost layer around the
+// box; ghost slots and the slots past the end of odd rows hold 0 and are never written).
+__device__ __forceinline__ unsigned rb_index(const RbDesc& d, int k, int y, int z) {
+    return (unsigned)(k + 1) + (unsigned)d.px * (unsigned)(y + 1) + d.pp * (unsigned)(z + 1);
+}
+
+// Compile-time integer, used to unroll a march with constant register indices.
+template <int N>
+struct IC {
+    static constexpr int value = N;
+};
+
+// Steps J .. N-1 of an unrolled stretch of a march over a register ring of length R:
+// f(IC<j mod R>, t + j) for each j, leaving the stretch (true) after the step of plane `last`.
+template <int J, int N, int R, class F>
+__device__ __forceinline__ bool ring_turn(F& f, int t, int last) {
+    if constexpr (J < N) {
+        f(IC<J % R>{}, t + J);
+        if (t + J >= last) return true;
+        return ring_turn<J + 1, N, R>(f, t, last);
+    } else {
+        return false;
+    }
 }
 
 }  // namespace

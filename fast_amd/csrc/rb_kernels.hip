@@ -10,12 +10,6 @@ namespace ft {
 // ---- red-black reduced system (mixed form, CG) --------------------------------------------
 namespace {
 
-// Element of slot k of row (y, z) in the padded per-colour layout (a ghost layer around the
-// box; ghost slots and the slots past the end of odd rows hold 0 and are never written).
-__device__ __forceinline__ unsigned rb_index(const RbDesc& d, int k, int y, int z) {
-    return (unsigned)(k + 1) + (unsigned)d.px * (unsigned)(y + 1) + d.pp * (unsigned)(z + 1);
-}
-
 // Position of a thread of an RB tile: slot k of row (y, z) of one colour, z marching.
 struct RbPos {
     int k, y, z0, z1;
@@ -130,13 +124,17 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
     double alpha = vs->alpha;   // U: replaced by this iteration's alpha below
     const double beta = vs->beta;
     const bool first = vs->first != 0;
-    const bool xpend = KIND == RB_P && vs->xpend == 2;   // uniform over the volume
+    // uniform over the volume: with the multigrid preconditioner z comes from its cycle (in the
+    // buffer this pass overwrites with p), so x takes one step every iteration
+    const bool mg = vs->mg != 0;
+    const bool xpend = KIND == RB_P && vs->xpend == (mg ? 1 : 2);
     const double xa0 = vs->xalpha[0], xa1 = vs->xalpha[1];
     const bool odd = (vs->phase & 1) != 0;
     const float* p_old = L.p[odd ? 1 : 0] + d.off_c;
     float* p_new = L.p[odd ? 0 : 1] + d.off_c;
     float* X = L.x + d.off_c;
     float* Rr = L.r + d.off_c;
+    const float* Za = (KIND == RB_P && mg) ? p_new : Rr;   // P: z, or r for z = D^-1 r
     float* Q = L.q + d.off_c;
     double* Y = L.y + d.off_c;
     const uint8_t* code_c = d.code_c[kColour];
@@ -151,11 +149,11 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
         const unsigned ci = valid(z, s, x) ? rb_index(d, ps.k, ps.y, z) : c00;
         in.code = ld(code_c, ci);
         if (KIND == RB_P) {
-            in.a = ld(Rr, ci);
+            in.a = ld(Za, ci);
             in.b = ld(p_old, ci);   // unused on the first iteration
             if (xpend) {
                 in.c = ld(X, ci);
-                in.e = ld(p_new, ci);   // p two iterations back, about to be overwritten
+                in.e = ld(p_new, ci);   // p two iterations back (or z), about to be overwritten
             }
         } else if (KIND == RB_Y) {
             rb_nbrs(p_new, d, ci, s, in.u);
@@ -178,10 +176,12 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
         const int bx = box_flags(x, ps.y, z, d.nx, d.ny, d.nz);
         const DiagInv<double> di = diag_at<double>(tabs.tab, code, bx, d.primary, c);
         if (KIND == RB_P) {
-            const double z_ = di.iv * (double)in.a;
+            const double z_ = mg ? (double)in.a : di.iv * (double)in.a;
             const double pn = first ? z_ : z_ + beta * (double)in.b;
             st(p_new, ci, (float)pn);
-            if (xpend) st(X, ci, (float)(((double)in.c + xa0 * (double)in.e) + xa1 * (double)in.b));
+            if (xpend)
+                st(X, ci, (float)(mg ? (double)in.c + xa0 * (double)in.b
+                                     : ((double)in.c + xa0 * (double)in.e) + xa1 * (double)in.b));
         } else if (KIND == RB_Y) {
             st(Y, ci, rb_sum(tabs.ftab, code, in.u) * di.iv);
         } else if (KIND == RB_Q) {
@@ -193,7 +193,10 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
             const float rs = (float)((double)in.c - alpha * (double)in.e);
             st(Rr, ci, rs);
             acc[0].add(rs, rs);
-            acc[1].add((double)rs, di.iv * (double)rs);
+            if (mg)
+                st(Q, ci, (float)(di.iv * (double)rs));   // x1 of the next cycle (q is spent)
+            else
+                acc[1].add((double)rs, di.iv * (double)rs);
         }
     };
     // loads AH planes ahead into a ring of AH + 1 register sets; no early exit: a step past
@@ -217,7 +220,7 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
         alpha = vs->absnew / pq;
         if (tile == d.tile_base && threadIdx.x == 0) {
             vs->alpha = alpha;
-            if (vs->xpend == 2) vs->xpend = 0;   // the P pass of this iteration added both steps
+            if (vs->xpend == (mg ? 1 : 2)) vs->xpend = 0;   // the P pass of this iteration added them
             if (!isfinite(alpha)) vs->status = ST_FRESH;
         }
         if (!isfinite(alpha)) return;
@@ -348,25 +351,6 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_q(RbLaunch L) {
         plane(z + 1, code_b, pv_b);
     }
     block_reduce_store<AccDD, 1, NT>(acc, L.part + (long long)tile * kPart);
-}
-
-// Compile-time integer, used to unroll the fused pass's march with constant register indices.
-template <int N>
-struct IC {
-    static constexpr int value = N;
-};
-
-// Steps J .. N-1 of an unrolled stretch of a march over a register ring of length R:
-// f(IC<j mod R>, t + j) for each j, leaving the stretch (true) after the step of plane `last`.
-template <int J, int N, int R, class F>
-__device__ __forceinline__ bool ring_turn(F& f, int t, int last) {
-    if constexpr (J < N) {
-        f(IC<J % R>{}, t + J);
-        if (t + J >= last) return true;
-        return ring_turn<J + 1, N, R>(f, t, last);
-    } else {
-        return false;
-    }
 }
 
 // Y and Q fused: q = S p = D_r p - A_rb (D_b^-1 A_br p) for a block's red tile without
@@ -576,6 +560,7 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
     constexpr int kColour = (KIND == RB_Y64) ? 1 : 0;
     const bool first_res = vs->refinements == 0;   // x64 not yet set: use x0
     const bool keep = vs->refinements > 0 && !vs->discard;
+    const bool mg = vs->mg != 0;
     // x lacks the steps of the last xpend iterations: the newest in the buffer the next P pass
     // reads as p_old, an older one in the other buffer; added in the P pass's order
     const int xpend = KIND == RB_UPD ? vs->xpend : 0;
@@ -660,6 +645,7 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
                 const double r64 = (b - di.d * xr) - rb_sum(tabs.ftab, code, o);
                 const float r32 = (float)r64;
                 st(Rr, ci, r32);
+                if (mg) st(L.q + d.off_c, ci, (float)(di.iv * (double)r32));   // x1 of the next cycle
                 acc[0].add(r64, r64);
                 acc[1].add(b, b);
                 acc[2].add(r32, r32);
@@ -699,7 +685,7 @@ __global__ __launch_bounds__(kFinThreads) void k_rb_fin(RbLaunch L) {
         double ta[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int k = 0; k < NP; ++k) ta[k] = tot[k];
-        if (FIN == F_CG1 && s->xpend == 2) s->xpend = 0;   // the P pass added both steps
+        if (FIN == F_CG1 && s->xpend == (s->mg ? 1 : 2)) s->xpend = 0;   // the P pass added them
         if (FIN == F_CG2) s->xalpha[s->xpend++] = s->alpha;   // x lacks this iteration's step
         fin_update<double, FIN>(s, ta);
     }
@@ -812,7 +798,11 @@ static void rb_launch_q(const RbLaunch& L, hipStream_t s) {
     rb_launch_it<RB_Q>(L, s);
 }
 
-hipError_t rb_iter(const RbLaunch& L, hipStream_t s) {
+hipError_t rb_iter(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {
+    if (M.nvol > 0) {
+        const hipError_t e = mg_cycle(L, M, s);
+        if (e != hipSuccess) return e;
+    }
     rb_launch_it<RB_P>(L, s);
     if (L.staged < 2) rb_launch_it<RB_Y>(L, s);   // the fused form computes Y itself
     rb_launch_q(L, s);

@@ -148,6 +148,16 @@ struct fast_server {
     double* d_xfull = nullptr;                // full-grid solutions of the finishing slots
     size_t xfull_cap = 0;
     RbLaunch RL{};
+    // multigrid preconditioner of the live set (slots whose extents take it)
+    MgLaunch ML{};
+    std::vector<MgDesc> h_mg;
+    MgDesc* d_mg = nullptr;
+    float* d_mgtab = nullptr;
+    double* d_mgpart = nullptr;
+    void* d_mglist = nullptr;                 // launch lists
+    size_t mgpart_cap = 0, mglist_cap = 0;
+    float* mg_base = nullptr;                 // level storage, 2 floats per arena element
+    void* mg_own = nullptr;                   // its own plane where the Y vector is in use
     int ntiles = 0;
 };
 
@@ -208,6 +218,10 @@ VolState<double> fresh_state(const fast_server* s, const Req* r) {
     v.delta2 = delta * delta;
     v.restart_cos = s->ctx->mixed_restart_cos;
     v.blowup2 = s->ctx->mixed_blowup2;
+    MgDesc plan;
+    size_t floats = 0;
+    v.mg = s->rb && mg_plan(r->nx, r->ny, r->nz, r->prm.dir / 2, &plan, &floats) ? 1 : 0;
+    v.mg_stall = s->ctx->mg_stall;
     v.eps2 = s->rb ? 2.220446049250313e-16 * 2.220446049250313e-16 : 1.1920928955078125e-07 * 1.1920928955078125e-07;
     return v;
 }
@@ -217,13 +231,21 @@ VolState<double> fresh_state(const fast_server* s, const Req* r) {
 int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     fast_ctx* ctx = s->ctx;
     int tiles = 0;
-    std::vector<int> tv;
+    std::vector<int> tv, mv;
+    int mg_tiles = 0;
     for (int i = 0; i < s->max_active; ++i) {
         RbDesc& d = s->h_rb[i];
         Req* r = s->slots[i];
         d = RbDesc{};
         d.tile_base = tiles;
         if (!r) continue;
+        size_t floats = 0;
+        if (mg_plan(r->nx, r->ny, r->nz, r->prm.dir / 2, &s->h_mg[i], &floats)) {
+            s->h_mg[i].part_base = mg_tiles;
+            s->h_mg[i].mem = s->mg_base + 2 * r->off;
+            mg_tiles += s->h_mg[i].ntiles;
+            mv.push_back(i);
+        }
         d.nx = r->nx;
         d.ny = r->ny;
         d.nz = r->nz;
@@ -251,6 +273,26 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     s->d_part = (double*)dalloc(ctx, s->tile_cap * 8 * sizeof(double));
     s->d_partb = (double*)dalloc(ctx, s->tile_cap * 8 * sizeof(double));
     if (!s->d_part || !s->d_partb) return FAST_E_OOM;
+    MgLists lists;
+    MgLaunch& M = s->ML;
+    mg_lists(s->h_mg, mv, &lists, &M);
+    std::vector<int> fresh;   // newly admitted: their levels are built below
+    for (Req* r : adm)
+        if (std::find(mv.begin(), mv.end(), r->slot) != mv.end()) fresh.push_back(r->slot);
+    if (M.nvol) {
+        const size_t b_vols = align_up(sizeof(int) * (mv.size() + fresh.size()), 256);
+        const size_t b_tiles = align_up(sizeof(int2) * lists.tiles.size(), 256);
+        if (!grow(s, (void**)&s->d_mgpart, &s->mgpart_cap, (size_t)mg_tiles, 2 * sizeof(double)) ||
+            !grow(s, &s->d_mglist, &s->mglist_cap, b_vols + b_tiles + sizeof(int2) * lists.blocks.size(), 1))
+            return FAST_E_OOM;
+        char* q = (char*)s->d_mglist;
+        M.vol = s->d_mg;
+        M.tab = s->d_mgtab;
+        M.part = s->d_mgpart;
+        M.vols = (const int*)q;
+        M.tiles = (const int2*)(q + b_vols);
+        M.blocks = (const int2*)(q + b_vols + b_tiles);
+    }
     hipStream_t st = ctx->stream;
     hipError_t e = hipStreamWaitEvent(st, s->up_done, 0);
     if (e == hipSuccess && tiles)
@@ -265,7 +307,14 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
         if (e == hipSuccess) e = hipMemcpyAsync(s->d_st + r->slot, &v, sizeof(v), hipMemcpyHostToDevice, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);   // c and v live on this stack frame
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(st);       // tv and h_rb are read by the copies
+    if (e == hipSuccess && M.nvol) {
+        e = hipMemcpyAsync(s->d_mg, s->h_mg.data(), sizeof(MgDesc) * s->max_active, hipMemcpyHostToDevice, st);
+        if (e == hipSuccess) e = mg_upload(M, lists, st);
+        if (e == hipSuccess && !fresh.empty())
+            e = hipMemcpyAsync(const_cast<int*>(M.vols) + mv.size(), fresh.data(), sizeof(int) * fresh.size(),
+                               hipMemcpyHostToDevice, st);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(st);       // tv, h_rb, h_mg and the lists are read by the copies
     if (!hip_ok(ctx, e, "server rebuild")) return FAST_E_HIP;
     RbLaunch& L = s->RL;
     L.ntiles = tiles;
@@ -293,7 +342,13 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     L.xfull = s->d_xfull;
     s->ntiles = tiles;
     if (!adm.empty()) {
-        const hipError_t et = ft::rb_setup(L, ctx->stream);   // tables of every slot, codes of the live set
+        hipError_t et = ft::rb_setup(L, ctx->stream);   // tables of every slot, codes of the live set
+        if (et == hipSuccess && !fresh.empty()) {
+            MgLaunch F = M;
+            F.vols = M.vols + mv.size();
+            F.nvol = (int)fresh.size();
+            et = ft::mg_setup(L, F, ctx->stream);
+        }
         if (!hip_ok(ctx, et, "server tables")) return FAST_E_HIP;
     }
     return FAST_OK;
@@ -546,7 +601,6 @@ void fail_all(fast_server* s, int rc) {
 void worker_main(fast_server* s) {
     fast_ctx* ctx = s->ctx;
     (void)hipSetDevice(ctx->device);
-    const int m = s->cfg.iters_per_round;
     for (;;) {
         std::vector<Req*> adm;
         {
@@ -580,10 +634,14 @@ void worker_main(fast_server* s) {
         // one round over the live set
         hipStream_t st = ctx->stream;
         hipError_t e = hipSuccess;
+        // preconditioned volumes need few and long iterations: short rounds, an update step each
+        const bool mg = s->rb && s->ML.nvol > 0;
+        const int m = mg ? std::min(s->cfg.iters_per_round, 4) : s->cfg.iters_per_round;
+        const int every = mg ? 1 : ctx->update_every;
         for (int i = 0; i < m && e == hipSuccess; ++i) {
-            const bool upd = (i + 1) % ctx->update_every == 0 || i + 1 == m;
+            const bool upd = (i + 1) % every == 0 || i + 1 == m;
             if (s->rb) {
-                e = ft::rb_iter(s->RL, st);
+                e = ft::rb_iter(s->RL, s->ML, st);
                 if (e == hipSuccess && upd) e = ft::rb_update(s->RL, st);
                 continue;
             }
@@ -645,7 +703,21 @@ int fast_server_create(fast_ctx* ctx, const fast_server_config* cfg, fast_server
     s->d_zero = (unsigned long long*)dalloc(ctx, sizeof(unsigned long long) * s->max_active);
     s->d_tab = (double*)dalloc(ctx, sizeof(double) * 2 * kTabEntries * s->max_active);
     s->d_rb = (RbDesc*)dalloc(ctx, sizeof(RbDesc) * s->max_active);
-    if (!s->arena_mem || !s->d_vol || !s->d_coef || !s->d_st || !s->d_zero || !s->d_tab || !s->d_rb ||
+    bool mg_ok = true;
+    if (s->rb) {
+        s->h_mg.assign(s->max_active, MgDesc{});
+        s->d_mg = (MgDesc*)dalloc(ctx, sizeof(MgDesc) * s->max_active);
+        s->d_mgtab = (float*)dalloc(ctx, sizeof(float) * kTabEntries * s->max_active);
+        mg_ok = s->d_mg && s->d_mgtab;
+        if (rb_mode() == 2) {   // the fused Y+Q pass stores no Y
+            s->mg_base = s->arena_mem ? (float*)rb_f64(s, 0) : nullptr;
+        } else {
+            s->mg_own = dalloc(ctx, s->S * 2 * sizeof(float));
+            s->mg_base = (float*)s->mg_own;
+            mg_ok = mg_ok && s->mg_own;
+        }
+    }
+    if (!mg_ok || !s->arena_mem || !s->d_vol || !s->d_coef || !s->d_st || !s->d_zero || !s->d_tab || !s->d_rb ||
         hipHostMalloc((void**)&s->h_st, sizeof(VolState<double>) * s->max_active, hipHostMallocDefault) != hipSuccess ||
         hipStreamCreateWithFlags(&s->up, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&s->up_done) != hipSuccess) {
         (void)hipGetLastError();
@@ -782,6 +854,11 @@ void fast_server_destroy(fast_server* s) {
     dfree(ctx, s->d_partb);
     dfree(ctx, s->d_tile_fin);
     dfree(ctx, s->d_xfull);
+    dfree(ctx, s->d_mg);
+    dfree(ctx, s->d_mgtab);
+    dfree(ctx, s->d_mgpart);
+    dfree(ctx, s->d_mglist);
+    dfree(ctx, s->mg_own);
     if (s->h_st) (void)hipHostFree(s->h_st);
     if (s->up_done) (void)hipEventDestroy(s->up_done);
     if (s->up) (void)hipStreamDestroy(s->up);

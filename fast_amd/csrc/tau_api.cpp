@@ -318,6 +318,7 @@ int fast_ctx_create(int device, size_t hbm_budget, fast_ctx** out) {
     if (const char* e = std::getenv("FAST_TAU_GRAPHS")) ctx->use_graphs = std::atoi(e) != 0;
     if (const char* e = std::getenv("FAST_TAU_GROUP_MB")) ctx->group_bytes = (size_t)std::atol(e) << 20;
     if (const char* e = std::getenv("FAST_TAU_UPDATE_EVERY")) ctx->update_every = std::max(1, std::atoi(e));
+    if (const char* e = std::getenv("FAST_TAU_MG_STALL")) ctx->mg_stall = std::max(1, std::atoi(e));
     *out = ctx;
     return FAST_OK;
 }
@@ -903,24 +904,71 @@ struct RbBatch {
     int* tile_vol_c = nullptr;   // compacted launch: volume and batch index of each live tile
     int* tile_id_c = nullptr;
     hipGraphExec_t gexec = nullptr;
+    // multigrid preconditioner
+    std::vector<MgDesc> hmg;     // by volume (nlev = 0: Jacobi)
+    std::vector<int> mg_vols;    // preconditioned volumes
+    MgLaunch M{};
+    void* mg_list = nullptr;     // launch lists on the device
+    void* mg_mem = nullptr;      // level storage where the Y vector is in use (separate Y and Q passes)
 
     ~RbBatch() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (ctx) {
             dfree(ctx, meta);
             dfree(ctx, vecs);
+            dfree(ctx, mg_list);
+            dfree(ctx, mg_mem);
         }
     }
 };
+
+void mg_lists(const std::vector<MgDesc>& desc, const std::vector<int>& vols, MgLists* out, MgLaunch* M) {
+    out->vols = vols;
+    out->tiles.clear();
+    out->blocks.clear();
+    M->nvol = (int)vols.size();
+    M->nlev = 0;
+    M->nlev_max = 0;
+    for (int v : vols) {
+        for (int t = 0; t < desc[v].ntiles; ++t) out->tiles.push_back(int2{v, t});
+        M->nlev = std::max(M->nlev, desc[v].bottom);
+        M->nlev_max = std::max(M->nlev_max, desc[v].nlev);
+    }
+    M->ntiles = (int)out->tiles.size();
+    for (int l = 0; l < M->nlev; ++l) {
+        M->blk_off[l] = (int)out->blocks.size();
+        for (int v : vols) {
+            if (l >= desc[v].bottom) continue;
+            const int nb = (int)((4ll * desc[v].lev[l + 1].n + kMgThreads - 1) / kMgThreads);
+            for (int b = 0; b < nb; ++b) out->blocks.push_back(int2{v, b});
+        }
+        M->nblk[l] = (int)out->blocks.size() - M->blk_off[l];
+    }
+}
+
+// The launch lists to the device (where M points).
+hipError_t mg_upload(const MgLaunch& M, const MgLists& l, hipStream_t s) {
+    auto up = [&](const void* dst, const void* src, size_t bytes) {
+        return bytes ? hipMemcpyAsync(const_cast<void*>(dst), src, bytes, hipMemcpyHostToDevice, s) : hipSuccess;
+    };
+    hipError_t e = up(M.vols, l.vols.data(), sizeof(int) * l.vols.size());
+    if (e == hipSuccess) e = up(M.tiles, l.tiles.data(), sizeof(int2) * l.tiles.size());
+    if (e == hipSuccess) e = up(M.blocks, l.blocks.data(), sizeof(int2) * l.blocks.size());
+    return e;
+}
 
 int rb_mode() {
     const char* e = std::getenv("FAST_TAU_RB_STAGED");
     return e ? std::min(2, std::max(0, std::atoi(e))) : 2;
 }
 
-static int prepare_rb(RbBatch& B) {
+static int prepare_rb(RbBatch& B, bool use_mg = true) {
     fast_ctx* ctx = B.ctx;
     const int nv = (int)B.jobs.size();
+    B.hmg.assign(nv, MgDesc{});
+    std::vector<size_t> mg_off(nv, 0);
+    size_t mg_floats = 0;
+    int mg_tiles = 0;
     B.hrb.resize(nv);
     B.hvol.resize(nv);
     B.hcoef.resize(nv);
@@ -990,6 +1038,16 @@ static int prepare_rb(RbBatch& B) {
         s.restart_cos = ctx->mixed_restart_cos;
         s.blowup2 = ctx->mixed_blowup2;
         s.solver = FAST_CG;
+        size_t floats = 0;
+        if (use_mg && mg_plan(v->nx, v->ny, v->nz, r.primary, &B.hmg[i], &floats)) {
+            s.mg = 1;
+            s.mg_stall = ctx->mg_stall;
+            B.hmg[i].part_base = mg_tiles;
+            mg_tiles += B.hmg[i].ntiles;
+            mg_off[i] = mg_floats;
+            mg_floats += align_up(floats, 64);
+            B.mg_vols.push_back(i);
+        }
     }
     B.ntiles = tiles;
     B.nplanes = planes;
@@ -1032,6 +1090,12 @@ static int prepare_rb(RbBatch& B) {
     o = align_up(o + sizeof(double) * planes, 256);
     const size_t o_tab = o;
     o = align_up(o + sizeof(double) * 2 * kTabEntries * nv, 256);
+    const size_t o_mg = o;
+    o = align_up(o + sizeof(MgDesc) * nv, 256);
+    const size_t o_mgpart = o;
+    o = align_up(o + sizeof(double) * 2 * (size_t)mg_tiles, 256);
+    const size_t o_mgtab = o;
+    o = align_up(o + sizeof(float) * kTabEntries * (mg_tiles ? nv : 0), 256);
     const size_t meta_bytes = o;
     // FP32 red vectors x, r, p[2], q (their region later holds the full-grid solution), then
     // FP64 y (black), x64 (red), x64b (black), then the per-colour codes
@@ -1094,7 +1158,31 @@ static int prepare_rb(RbBatch& B) {
     }
     e = hipMemcpyAsync(m + o_rb, B.hrb.data(), sizeof(RbDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = ft::rb_setup(L, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);   // hrb is read by the copy
+    MgLists lists;
+    if (!B.mg_vols.empty()) {
+        // the fused Y+Q pass stores no Y: the levels take its place (8 bytes per padded element,
+        // at most 2 floats of which they need, see mg_plan)
+        MgLaunch& M = B.M;
+        if (L.staged != 2) B.mg_mem = dalloc(ctx, mg_floats * sizeof(float));
+        float* mem = L.staged == 2 ? (float*)L.y : (float*)B.mg_mem;
+        for (int i : B.mg_vols) B.hmg[i].mem = L.staged == 2 ? mem + 2 * B.hrb[i].off_c : mem + mg_off[i];
+        mg_lists(B.hmg, B.mg_vols, &lists, &M);
+        const size_t b_vols = align_up(sizeof(int) * lists.vols.size(), 256);
+        const size_t b_tiles = align_up(sizeof(int2) * lists.tiles.size(), 256);
+        B.mg_list = dalloc(ctx, b_vols + b_tiles + sizeof(int2) * lists.blocks.size());
+        if (!mem || !B.mg_list) return FAST_E_OOM;
+        char* q = (char*)B.mg_list;
+        M.vol = (const MgDesc*)(m + o_mg);
+        M.part = (double*)(m + o_mgpart);
+        M.tab = (float*)(m + o_mgtab);
+        M.vols = (const int*)q;
+        M.tiles = (const int2*)(q + b_vols);
+        M.blocks = (const int2*)(q + b_vols + b_tiles);
+        if (e == hipSuccess) e = hipMemcpyAsync(m + o_mg, B.hmg.data(), sizeof(MgDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
+        if (e == hipSuccess) e = mg_upload(M, lists, ctx->stream);
+        if (e == hipSuccess) e = ft::mg_setup(L, M, ctx->stream);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);   // the copies read hrb, hmg and the lists
     return hip_ok(ctx, e, "diagonal tables") ? FAST_OK : FAST_E_HIP;
 }
 
@@ -1114,13 +1202,15 @@ static int solve_mixed_rb(fast_ctx* ctx, std::vector<Job*>& jobs) {
     if (!hip_ok(ctx, e, "mixed init")) return FAST_E_HIP;
     long maxit = 0;
     for (auto* j : jobs) maxit = std::max(maxit, j->prm.max_iter);
-    const int chunk = ctx->chunk;
+    // preconditioned iterations are few and long: short polling rounds, an update step each
+    int chunk = B.M.nvol > 0 ? std::min(ctx->chunk, 4) : ctx->chunk;
+    int every = B.M.nvol > 0 ? 1 : ctx->update_every;
     const long max_chunks = 3 * (maxit / chunk + 2) + 16;
     auto round = [&]() -> hipError_t {
         hipError_t e2 = hipSuccess;
         for (int i = 0; i < chunk && e2 == hipSuccess; ++i) {
-            e2 = ft::rb_iter(B.L, s);
-            const bool upd = (i + 1) % ctx->update_every == 0 || i + 1 == chunk;
+            e2 = ft::rb_iter(B.L, B.M, s);
+            const bool upd = (i + 1) % every == 0 || i + 1 == chunk;
             if (e2 == hipSuccess && upd) e2 = ft::rb_update(B.L, s);
         }
         return e2;
@@ -1130,7 +1220,20 @@ static int solve_mixed_rb(fast_ctx* ctx, std::vector<Job*>& jobs) {
     // Batch tails: once the unfinished volumes hold at most half of the launched tiles, later
     // rounds launch only theirs (a captured round is replaced by a new capture).
     const RbLaunch full = B.L;
+    auto drop_graph = [&] {
+        if (B.gexec) (void)hipGraphExecDestroy(B.gexec);
+        B.gexec = nullptr;
+    };
     auto poll = [&](const VolState<double>* snap) -> hipError_t {
+        // once no unfinished volume is preconditioned any more: rounds of the Jacobi form
+        bool mg = false;
+        for (int i : B.mg_vols) mg = mg || (snap[i].status != ST_IDLE && snap[i].mg);
+        if (!mg && B.M.nvol > 0) {
+            B.M.nvol = 0;
+            chunk = ctx->chunk;
+            every = ctx->update_every;
+            drop_graph();
+        }
         long live = 0;
         for (size_t i = 0; i < jobs.size(); ++i)
             if (snap[i].status != ST_IDLE) live += B.hrb[i].ntiles;
@@ -1150,10 +1253,16 @@ static int solve_mixed_rb(fast_ctx* ctx, std::vector<Job*>& jobs) {
         B.L.tile_vol = B.tile_vol_c;
         B.L.tile_id = B.tile_id_c;
         B.L.ntiles = (int)live;
-        if (B.gexec) {
-            (void)hipGraphExecDestroy(B.gexec);
-            B.gexec = nullptr;
+        if (B.M.nvol > 0) {
+            std::vector<int> mv;
+            for (int i : B.mg_vols)
+                if (snap[i].status != ST_IDLE) mv.push_back(i);
+            MgLists lists;
+            mg_lists(B.hmg, mv, &lists, &B.M);
+            if (e2 == hipSuccess) e2 = mg_upload(B.M, lists, s);
+            if (e2 == hipSuccess) e2 = hipStreamSynchronize(s);   // the copies read the lists
         }
+        drop_graph();
         return e2;
     };
     rc = drive(B, ST_IDLE, max_chunks, step, restart, poll);
@@ -1444,17 +1553,17 @@ static int time_rb_passes(fast_volume* vol, int dir, int iters, double* ms) {
     RbBatch B;
     B.ctx = ctx;
     B.jobs = {&j};
-    int rc = prepare_rb(B);
+    int rc = prepare_rb(B, false);   // the passes of the Jacobi form
     if (rc) return rc;
     hipStream_t s = ctx->stream;
     hipEvent_t ev[2];
     (void)hipEventCreate(&ev[0]);
     (void)hipEventCreate(&ev[1]);
     hipError_t e = ft::rb_update(B.L, s);
-    for (int i = 0; i < 2 && e == hipSuccess; ++i) e = ft::rb_iter(B.L, s);
+    for (int i = 0; i < 2 && e == hipSuccess; ++i) e = ft::rb_iter(B.L, B.M, s);
     for (int k = 0; k < 5 && e == hipSuccess; ++k) {
         e = hipEventRecord(ev[0], s);
-        for (int i = 0; i < iters && e == hipSuccess; ++i) e = k == 4 ? ft::rb_iter(B.L, s) : ft::rb_pass_only(B.L, k, s);
+        for (int i = 0; i < iters && e == hipSuccess; ++i) e = k == 4 ? ft::rb_iter(B.L, B.M, s) : ft::rb_pass_only(B.L, k, s);
         if (e == hipSuccess) e = hipEventRecord(ev[1], s);
         if (e == hipSuccess) e = hipEventSynchronize(ev[1]);
         float t = 0;

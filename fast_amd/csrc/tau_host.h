@@ -69,6 +69,7 @@ struct fast_ctx {
     bool use_graphs = true;                    // replay polling rounds from a captured HIP graph
     size_t group_bytes = (size_t)320 << 20;    // red-black batches: state bytes per sub-batch (0 = one launch)
     int update_every = fth::kMixedUpdateEvery; // mixed form: iterations between reliable-update steps
+    int mg_stall = ft::kMgStall;               // preconditioned CG: iterations without an update before the Jacobi form
     // mixed BiCGSTAB: reset r0 = r when r0 and r are this close to orthogonal (0: only by
     // Eigen's rule), and drop the correction when |r|^2 grows this much since the last update
     // (infinite: only a non-finite residual does)
@@ -126,6 +127,14 @@ RbShape rb_shape(const fast_ctx* ctx, int nx, int ny, int nz);
 int rb_tz(int hx, int ny, int nz, int ty);
 std::string rb_key(int nx, int ny, int nz);
 bool rb_ty_compiled(int ty);
+// Launch lists of the multigrid cycle over the preconditioned volumes `vols` (indices into
+// `desc`): their fine tiles and the blocks of their block-wise levels, and the counts of M.
+struct MgLists {
+    std::vector<int> vols;
+    std::vector<int2> tiles, blocks;
+};
+void mg_lists(const std::vector<ft::MgDesc>& desc, const std::vector<int>& vols, MgLists* out, ft::MgLaunch* M);
+hipError_t mg_upload(const ft::MgLaunch& M, const MgLists& lists, hipStream_t s);
 // Form of the red-black Y and Q passes (RbLaunch::staged): FAST_TAU_RB_STAGED = 0 (separate,
 // Q reads six Y values), 1 (separate, Q stages the Y planes in LDS), default 2 (fused).
 int rb_mode();

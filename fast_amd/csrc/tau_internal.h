@@ -61,6 +61,10 @@ struct VolState {
     int xpend;                     // red-black CG: steps alpha p that x still lacks (0..2), the
                                    // last xpend iterations'; the P pass adds two, the update any
     double xalpha[2];              // their alphas, oldest first
+    int mg;                        // red-black CG: multigrid preconditioner (MgDesc) instead of Jacobi; x then
+                                   // takes its step every iteration (xpend 0..1)
+    int mg_since, mg_stall;        // its iterations since the last reliable update, and their limit
+    int pad;
 };
 
 // Vectors of one (batched) solve, concatenated over its volumes (element offset VolDesc::off).
@@ -218,10 +222,64 @@ constexpr int kRbTX = 64;   // threads per block along k (one wave per row of a 
 // holds the same four slots of a row in every plane.
 inline int rb_row_pitch(int hx) { return (hx + 2 + 3) & ~3; }
 
+// Multigrid preconditioner of the red-black CG.  z = B r, B the red-red block of one V-cycle
+// for the full system A, started from zero with the red residual (the black one is 0):
+//   fine level: Gauss-Seidel red then black, coarse correction, black then red;
+//   coarse levels: cells of 2 x 2 x 2 children (an axis of one cell stays), piecewise constant
+//   transfer, the Galerkin operator's face coefficients (sums of the children's faces) times
+//   1/2, which is the coarse cells' area over their distance; the same sweeps.
+// The cycle is symmetric, so CG applies.  On the fine level everything is expressed in
+// x1 = D_r^-1 r: a red sweep from zero gives x1, the black one -Y(x1) = -D_b^-1 A_br x1, the
+// residual left on the red voxels is A_rb Y(x1), and after the correction x2 = x1 + P e the last
+// two sweeps give z = D_r^-1 (r + A_rb Y(x2)).  None of these sums cancels, so the cycle runs in
+// FP32; the CG around it keeps its FP64 arithmetic, FP64 residuals and stopping rule.
+// A volume whose residual has not dropped to its next reliable update within kMgStall iterations
+// (seen at solid conductivities of 1e-6 and 95% solid) goes on with the Jacobi form from its x64.
+// Level l >= 1 holds, per cell, the right-hand side (overwritten by the solution), the black
+// values of the first sweep, the face coefficients towards x+, y+ and z+, and 1 / diagonal, all
+// for -A (positive).  Levels from `bottom` on are solved by one block per volume in LDS.
+constexpr int kMgStall = 128;           // iterations without a reliable update before the Jacobi form takes over
+constexpr int kMgLevels = 20;           // levels of the coarsest hierarchy a solver volume can have
+constexpr int kMgArrays = 6;            // g, t, cx, cy, cz, iv
+constexpr int kMgBottomCells = 5120;    // cells of the levels the one-block kernel keeps in LDS
+constexpr int kMgTY = 8;                // rows per fine tile (even: a tile holds whole coarse cells)
+constexpr int kMgThreads = 256;         // threads of a coarse-level block (4 per coarse cell)
+struct MgLevel {
+    int nx, ny, nz, n;
+    unsigned off;                       // floats from MgDesc::mem to the level's arrays
+};
+struct MgDesc {
+    int nlev, bottom;                   // coarse levels (lev[0] is the fine grid's first coarsening)
+    int tiles_x, tiles_y, tiles_z, tz;  // fine tiles of 64 slots x kMgTY rows x tz planes (tz even)
+    int ntiles, part_base;
+    float* mem;
+    MgLevel lev[kMgLevels];
+};
+struct MgLaunch {
+    int nvol, ntiles;                   // preconditioned volumes, fine tiles
+    int nlev, nlev_max;                 // levels launched block-wise; most levels of a volume
+    const MgDesc* vol;                  // by volume of the batch
+    const int* vols;                    // the preconditioned volumes
+    const int2* tiles;                  // fine tiles: (volume, tile of the volume)
+    const int2* blocks;                 // coarse-level blocks: (volume, block of its level), level after level
+    int blk_off[kMgLevels], nblk[kMgLevels];
+    double* part;                       // 2 doubles per fine tile: r.z as (hi, lo)
+    float* tab;                         // per volume kTabEntries: -1 / diagonal
+};
+// Level geometry of an nx x ny x nz volume with flow along axis `primary`; false where it takes
+// the Jacobi form (the rule depends on the extents alone).  Fills everything but part_base and mem; *floats: level
+// storage, at most 2 floats per element of the padded per-colour layout.
+bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats);
+// Level coefficients and FP32 tables (codes and Coef uploaded before).
+hipError_t mg_setup(const RbLaunch&, const MgLaunch&, hipStream_t);
+// z = B r into the buffer of the next p, then beta, for the running volumes that are preconditioned.
+hipError_t mg_cycle(const RbLaunch&, const MgLaunch&, hipStream_t);
+
 // Diagonal tables and per-colour codes (after the vectors and codes were zero-filled).
 hipError_t rb_setup(const RbLaunch&, hipStream_t);
-// One CG iteration on S for the volumes in ST_RUNNING (4 passes, 2 per-volume finalizes).
-hipError_t rb_iter(const RbLaunch&, hipStream_t);
+// One CG iteration on S for the volumes in ST_RUNNING (4 passes, 2 per-volume finalizes; the
+// cycle first where volumes are preconditioned).
+hipError_t rb_iter(const RbLaunch&, const MgLaunch&, hipStream_t);
 // Reliable update / start for the volumes in ST_UPDATE or ST_FRESH: x64 += x, x = 0, then the
 // FP64 residual r = b_S - S x64 (x64 = x0 on the first step) and the FP64 convergence test.
 hipError_t rb_update(const RbLaunch&, hipStream_t);

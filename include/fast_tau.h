@@ -69,8 +69,10 @@ typedef struct fast_tau_params {
     double mixed_inner_tol; /* MIXED only: residual reduction between FP64 reliable updates (0 = 0.1) */
     double mixed_outer_tol; /* MIXED only: FP64 true relative residual target (0 = `tolerance`) */
     int verbose;
-    int mixed_full_grid;  /* MIXED + CG only: 0 (default) = CG on the red-black Schur complement
-                             (about half the iterations); 1 = CG on the full grid */
+    int mixed_full_grid;  /* MIXED + CG only: 0 (default) = CG on the red-black Schur complement, with a
+                             multigrid preconditioner from 98304 voxels and 24 along the flow on
+                             (a tenth of the iterations), else Jacobi (half of them); 1 = CG on
+                             the full grid */
     int flux_nonuniform;  /* TortuosityParams::useNonUniform (VolumeMeasures.h:27): the flux sums
                              pore voxels only, with half spacing towards a solid neighbour, and a
                              plane's mean divides by its pore count (VolumeMeasures.cpp:228-264) */
@@ -113,6 +115,8 @@ typedef struct fast_ctx fast_ctx;
  * FAST_TAU_UPDATE_EVERY (default 4) is the number of mixed-form iterations between launches of
  * the reliable-update step (results are the same for every value); FAST_TAU_RB_TZ forces the
  * z depth of the red-black tiles (default: nz * tiles per plane / 2048, clamped to 4..32);
+ * FAST_TAU_MG_STALL (default 128) is the number of multigrid-preconditioned iterations without a
+ * reliable update after which a mixed CG solve goes on with the Jacobi preconditioner;
  * FAST_TAU_RB_STAGED=0 selects the red-black Q pass that reads its Y neighbours from memory
  * instead of staging them in LDS (results are bit-identical). */
 int fast_ctx_create(int device, size_t hbm_budget, fast_ctx** out);
@@ -254,7 +258,8 @@ typedef struct fast_server_config {
                              per-colour layout, (ceil(nx/2)+2)(ny+2)(nz+2) elements (about
                              23 B per voxel), with CG; 56 B per voxel with BiCGSTAB */
     int max_active;         /* max concurrently solving requests (0 = 64) */
-    int iters_per_round;    /* Krylov iterations between admission points (0 = 8) */
+    int iters_per_round;    /* Krylov iterations between admission points (0 = 8; at most 4 while a
+                               multigrid-preconditioned request is live) */
     int use_bicgstab;       /* 0: CG (default), 1: BiCGSTAB */
     int reserved[3];
 } fast_server_config;
