@@ -1,6 +1,7 @@
 """Autotuner of the tile shapes per volume size class.
 
-Full grid (FP64 and FP32/mixed BiCGSTAB, mixed CG with mixed_full_grid): for every size
+Full grid (FP64 and FP32/mixed BiCGSTAB, mixed CG with mixed_full_grid; only with --classes,
+since the library's own rule looks at a volume's extents rather than its class): for every size
 class (per-axis edge class 32/64/128/256/512, precision) it times one Krylov iteration of
 the solver that precision mostly runs (FP64: BiCGSTAB, mixed: CG) with HIP events for every
 compiled block shape (tx x ty) and a range of tz, and writes the fastest as lines
@@ -15,7 +16,7 @@ The lines go to tuning_gfx950.txt next to libfasttau.so, where the library picks
 (or wherever $FAST_TAU_TUNING points).  Tile shapes never change results: every dot product
 is rounded once from a double-double sum.
 
-  python -m fast_amd.autotune [--classes 32,64,128,256] [--rb-classes 32,...,512] [--out PATH]
+  python -m fast_amd.autotune [--classes 32,...] [--rb-classes 32,...,512] [--out PATH]
 """
 from __future__ import annotations
 
@@ -149,7 +150,7 @@ def write_table(out: Path, grid: dict, rb: dict) -> None:
 
 def main() -> int:
     ap = argparse.ArgumentParser()
-    ap.add_argument("--classes", default="32,64,128,256", help="full-grid size classes ('' to skip)")
+    ap.add_argument("--classes", default="", help="full-grid size classes")
     ap.add_argument("--rb-classes", default="32,64,128,256,512", help="red-black size classes ('' to skip)")
     ap.add_argument("--out", default=str(LIB_PATH.parent / "tuning_gfx950.txt"))
     ap.add_argument("--iters", type=int, default=12)

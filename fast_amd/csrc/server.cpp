@@ -772,7 +772,9 @@ int fast_server_submit(fast_server* s, const uint8_t* mask, int nx, int ny, int 
         r->tz = rb_shape(s->ctx, nx, ny, nz).tz;
     } else {
         r->elems = align_up(n, kAlign);
-        r->tz = choose_shape(nx, ny, nz, FAST_MIXED, s->ctx).tz;
+        // planes per 64 x 8 tile: many requests share a launch, so a volume alone need not fill the chip
+        const long long txy = (long long)((nx + kTX - 1) / kTX) * ((ny + kTY - 1) / kTY);
+        r->tz = (int)std::max<long long>(8, std::min<long long>(32, (long long)nz * txy / 1024));
     }
     {
         std::lock_guard<std::mutex> lk(s->mu);

@@ -161,30 +161,62 @@ Coef<T> make_coef(int nx, int ny, int nz, int dir, double d_pore, double d_solid
 template Coef<double> make_coef<double>(int, int, int, int, double, double);
 template Coef<float> make_coef<float>(int, int, int, int, double, double);
 
-// Tile shape: the block is TX x TY threads; TX follows the x extent so short rows do not
-// leave lanes idle.  tz (planes per tile) is chosen from the volume alone so that a large
-// volume yields ~2048+ tiles.  Both depend only on the volume, which keeps per-volume
-// reductions independent of the batch.
 static bool shape_compiled(int tx, int ty) {
     return (tx == 64 && (ty == 4 || ty == 8 || ty == 16)) || (tx == 32 && (ty == 8 || ty == 16 || ty == 32)) ||
            (tx == 16 && ty == 16);
 }
 
-Shape choose_shape(int nx, int ny, int nz, int precision, const fast_ctx* ctx) {
-    Shape s{64, 8, 16};
+// Tile shape of the full-grid passes over one or several volumes: the block shape and planes per
+// tile with the least modelled time.  The tiles run in rounds of as many blocks as 256 CUs hold: 16
+// waves each in FP64 (112 VGPRs) and in the mixed form, 24 in FP32.  A round takes its planes per
+// tile and a prologue of one or two; a plane costs the same up to 12 waves on a CU (18 with 4-byte
+// vectors) and grows with the waves beyond.  Among equals the larger block wins in FP64 (fewer halo rows), 64x8
+// where vectors take 4 bytes.  What decides at ordinary sizes is the last round: 191 x 205 x 177 in
+// the best 256^3 shape, 64x16x64, is 117 tiles for 256 CUs.  Measured over 14 extents, FP64 and FP32,
+// against sweeps of all shapes: within 3-4% of the best on average and 10% at most, where one
+// shape per power-of-two size class was up to 2.3x off (FP64 CG, an iteration: 160x150x140 148 -> 63
+// us, 191x205x177 168 -> 108, 100^3 53 -> 41, 256^3 243 both).
+static Shape model_shape(const std::vector<const fast_volume*>& vols, int precision) {
+    static const int kBySize[][2] = {{64, 16}, {64, 8}, {32, 32}, {32, 16}, {64, 4}, {32, 8}, {16, 16}};
+    static const int k64x8[][2] = {{64, 8}, {64, 16}, {32, 16}, {32, 32}, {64, 4}, {32, 8}, {16, 16}};
+    const bool fp64 = precision == FAST_FP64;
+    const int held = precision == FAST_FP32 ? 24 : 16, prologue = fp64 ? 1 : 2;
+    const double keeps_up = fp64 ? 12.0 : 18.0;   // waves on a CU beyond which a plane takes longer
+    int nzmax = 1;
+    for (const fast_volume* v : vols) nzmax = std::max(nzmax, v->nz);
+    Shape best{64, 8, 16};
+    double least = HUGE_VAL;
+    for (const auto& s : fp64 ? kBySize : k64x8) {
+        const int waves = s[0] * s[1] / 64;
+        const long long cap = 256 * (held / waves);
+        int last = 0;
+        for (int n = 1; n <= nzmax; ++n) {   // tiles along z of the deepest volume
+            const int tz = (nzmax + n - 1) / n;
+            if (tz == last || tz > 64 || (tz < 2 && nzmax > 1)) continue;
+            last = tz;
+            long long tiles = 0;
+            for (const fast_volume* v : vols)
+                tiles += (long long)((v->nx + s[0] - 1) / s[0]) * ((v->ny + s[1] - 1) / s[1]) * ((v->nz + tz - 1) / tz);
+            auto plane = [&](long long blocks) { return std::max(1.0, (double)(blocks * waves) / keeps_up); };
+            const long long rest = tiles % cap;
+            const double t = (tz + prologue) *
+                             ((double)(tiles / cap) * plane(held / waves) + (rest ? plane((rest + 255) / 256) : 0.0));
+            if (t < least) {
+                least = t;
+                best = Shape{s[0], s[1], tz};
+            }
+        }
+    }
+    return best;
+}
+
+Shape choose_shape(const std::vector<const fast_volume*>& vols, int precision, const fast_ctx* ctx) {
     if (ctx->forced.tx) return ctx->forced;
-    const auto key = shape_key(nx, ny, nz, precision);
-    auto it = ctx->tuned.find(key);
-    if (it != ctx->tuned.end()) return it->second;
-    if (nx <= 16)
-        s = {16, 16, 16};
-    else if (nx <= 32)
-        s = {32, 8, 16};
-    const long long txy = (long long)((nx + s.tx - 1) / s.tx) * ((ny + s.ty - 1) / s.ty);
-    long long tz = (long long)nz * txy / 2048;
-    tz = std::max<long long>(8, std::min<long long>(32, tz));
-    s.tz = (int)tz;
-    return s;
+    const fast_volume* big = vols[0];
+    for (const fast_volume* v : vols)
+        if ((size_t)v->nx * v->ny * v->nz > (size_t)big->nx * big->ny * big->nz) big = v;
+    auto it = ctx->tuned.find(shape_key(big->nx, big->ny, big->nz, precision));
+    return it != ctx->tuned.end() ? it->second : model_shape(vols, precision);
 }
 
 // Tuned tile shapes: text lines "<size-class key> <tx> <ty> <tz>" written by the autotuner
@@ -1304,14 +1336,10 @@ int solve_jobs(fast_ctx* ctx, std::vector<Job>& jobs) {
         j.porosity = (p.porosity >= 0) ? p.porosity : (double)(float)((double)j.vol->zeros / (double)n);
         j.update_delta = (p.mixed_inner_tol > 0 && p.mixed_inner_tol < 1) ? p.mixed_inner_tol : 0.1;
         j.outer_tol = p.mixed_outer_tol > 0 ? p.mixed_outer_tol : p.tolerance;
-        const Shape sh = choose_shape(j.vol->nx, j.vol->ny, j.vol->nz, p.precision, ctx);
-        j.tz = sh.tz;
-        j.shape = sh;
         std::memset(j.res, 0, sizeof(*j.res));
         j.res->true_rel_residual = -1;
     }
-    // one batched solve per (precision, solver); its block shape is the one chosen for the
-    // largest volume (results do not depend on the tile shape), each volume keeps its own tz
+    // one batched solve per (precision, solver), one tile shape each (results do not depend on it)
     std::map<std::tuple<int, int, int>, std::vector<Job*>> groups;
     for (auto& j : jobs) {
         const int rb = j.prm.precision == FAST_MIXED && j.prm.solver == FAST_CG && !j.prm.mixed_full_grid;
@@ -1354,10 +1382,10 @@ int solve_jobs(fast_ctx* ctx, std::vector<Job>& jobs) {
             if (rc) return rc;
             continue;
         }
-        const Job* big = g.second[0];
-        for (const Job* j : g.second)
-            if ((size_t)j->vol->nx * j->vol->ny * j->vol->nz > (size_t)big->vol->nx * big->vol->ny * big->vol->nz) big = j;
-        const Shape sh{big->shape.tx, big->shape.ty, 16};
+        std::vector<const fast_volume*> vols;
+        for (const Job* j : g.second) vols.push_back(j->vol);
+        const Shape sh = choose_shape(vols, prec, ctx);
+        for (Job* j : g.second) j->tz = sh.tz;
         int rc;
         if (prec == FAST_FP64)
             rc = solve_plain<double, double>(ctx, g.second, sh, solver);
@@ -1444,7 +1472,7 @@ static int debug_apply(fast_volume* vol, int dir, const T* x, T* y) {
     j.prm.dir = dir;
     fast_tau_result res;
     j.res = &res;
-    const Shape sh = choose_shape(vol->nx, vol->ny, vol->nz, sizeof(T) == 8 ? FAST_FP64 : FAST_FP32, ctx);
+    const Shape sh = choose_shape({vol}, sizeof(T) == 8 ? FAST_FP64 : FAST_FP32, ctx);
     j.tz = sh.tz;
     Batch<T, T> B;
     B.ctx = ctx;
@@ -1479,7 +1507,7 @@ static int time_passes(fast_volume* vol, int dir, int solver, int iters, double*
     j.prm.max_iter = 1L << 40;
     fast_tau_result res;
     j.res = &res;
-    const Shape sh = choose_shape(vol->nx, vol->ny, vol->nz, sizeof(T) == 8 ? FAST_FP64 : FAST_MIXED, ctx);
+    const Shape sh = choose_shape({vol}, sizeof(T) == 8 ? FAST_FP64 : FAST_MIXED, ctx);
     j.tz = sh.tz;
     Batch<T, A> B;
     B.ctx = ctx;
@@ -1645,7 +1673,7 @@ int fast_debug_system_f64(fast_volume* vol, int dir, double* b, double* x0, doub
         j.prm.solver = FAST_CG;
         fast_tau_result res;
         j.res = &res;
-        const Shape sh = choose_shape(vol->nx, vol->ny, vol->nz, FAST_FP64, ctx);
+        const Shape sh = choose_shape({vol}, FAST_FP64, ctx);
         j.tz = sh.tz;
         Batch<double, double> B;
         B.ctx = ctx;

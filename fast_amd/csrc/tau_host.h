@@ -100,7 +100,6 @@ struct Job {
     double porosity = 0;
     double update_delta = 0.1, outer_tol = 0;
     int tz = 16;
-    Shape shape{64, 8, 16};
 };
 
 // CCL on the volume's mask (ccl_api.cpp): labels cached on the volume per background value
@@ -116,7 +115,7 @@ bool hip_ok(fast_ctx* ctx, hipError_t e, const char* what);
 template <class T>
 ft::Coef<T> make_coef(int nx, int ny, int nz, int dir, double d_pore, double d_solid);
 std::string shape_key(int nx, int ny, int nz, int precision);
-Shape choose_shape(int nx, int ny, int nz, int precision, const fast_ctx* ctx);
+Shape choose_shape(const std::vector<const fast_volume*>& vols, int precision, const fast_ctx* ctx);
 void load_tuning(fast_ctx* ctx);
 int solve_jobs(fast_ctx* ctx, std::vector<Job>& jobs);
 // Red-black tile shape of a volume: forced (fast_ctx_set_rb_shape), else the tuned entry of
