@@ -226,12 +226,24 @@ __device__ __forceinline__ void block_reduce_store(Acc (&acc)[NP], double* out) 
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    // the waves' sums by 16 lanes per accumulator (one thread adding up to 16 of them in turn is a
+    // chain of 160 FP64 operations at the end of every pass)
+    static_assert(NW <= 16 && NP <= 4, "one lane per wave and accumulator");
+    if (w == 0) {
+        const int k = lane >> 4, i = lane & 15;
+        Acc a;
+        a.init();
+        if (k < NP && i < NW) {
+            a.hi = red[i][k][0];
+            a.lo = red[i][k][1];
+        }
 #pragma unroll
-        for (int k = 0; k < NP; ++k) {
-            Acc a;
-            a.init();
-            for (int i = 0; i < NW; ++i) a.add2(red[i][k][0], red[i][k][1]);
+        for (int off = NW > 8 ? 8 : (NW > 4 ? 4 : (NW > 2 ? 2 : 1)); off > 0; off >>= 1) {
+            const double h = __shfl_xor(a.hi, off, 64);
+            const double l = __shfl_xor(a.lo, off, 64);
+            a.add2(h, l);
+        }
+        if (k < NP && i == 0) {
             out[2 * k] = a.hi;
             out[2 * k + 1] = a.lo;
         }
@@ -285,10 +297,39 @@ __device__ __forceinline__ void reduce_volume(const double* part, int base, int 
 #pragma unroll
             for (int k = 0; k < NP; ++k) sums[k].add2(v[u][2 * k], v[u][2 * k + 1]);
     }
-    block_reduce_store<AccDD, NP, NT>(sums, red);
+    block_reduce_store<AccDD, NP, NT>(sums, red);   // written by the first wave, read by it
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int k = 0; k < NP; ++k) tot[k] = red[2 * k] + red[2 * k + 1];
+    }
+}
+
+// The same by the first wave of the block alone (no barrier): thread 0 gets the totals.
+template <int NP>
+__device__ __forceinline__ void reduce_volume_wave(const double* part, int base, int n, double (&tot)[NP]) {
+    if (threadIdx.x >= 64) return;
+    AccDD sums[NP];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) sums[k].init();
+    constexpr int U = 4;   // tiles in flight per lane
+    for (int t0 = (int)threadIdx.x; t0 < n; t0 += U * 64) {
+        double v[U][2 * NP];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = t0 + u * 64;
+            const double* p = part + (long long)(base + (t < n ? t : 0)) * kPart;
+#pragma unroll
+            for (int k = 0; k < 2 * NP; ++k) v[u][k] = (t < n) ? p[k] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < NP; ++k) sums[k].add2(v[u][2 * k], v[u][2 * k + 1]);
+    }
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        wave_combine(sums[k]);
+        tot[k] = sums[k].hi + sums[k].lo;
     }
 }
 

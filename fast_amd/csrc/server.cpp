@@ -413,10 +413,15 @@ int rebuild(fast_server* s, const std::vector<Req*>& adm) {
     L.ty = kTY;
     L.ntiles = tiles;
     L.nvol = s->max_active;
+    if (const Req* r = s->slots[0]) {   // read by launches over one slot (max_active = 1)
+        L.vol0 = s->h_vol[0];
+        L.coef0 = make_coef<double>(r->nx, r->ny, r->nz, r->prm.dir, r->prm.d_pore, r->prm.d_solid);
+    }
     L.vol = s->d_vol;
     L.tile_vol = s->d_tile;
     L.coef = s->d_coef;
     L.st = s->d_st;
+    L.st_out = s->d_st;
     L.part = s->d_part;
     L.tab = s->d_tab;
     float* a = (float*)s->arena_mem;

@@ -636,6 +636,8 @@ static int prepare(Batch<T, A>& B) {
     o = align_up(o + sizeof(Coef<double>) * nv, 256);
     const size_t o_st = o;
     o = align_up(o + sizeof(VolState<A>) * nv, 256);
+    const size_t o_st2 = o;
+    o = align_up(o + sizeof(VolState<A>) * nv, 256);
     const size_t o_tile = o;
     o = align_up(o + sizeof(int) * tiles, 256);
     const size_t o_part = o;
@@ -674,10 +676,15 @@ static int prepare(Batch<T, A>& B) {
     B.L.ty = B.shape.ty;
     B.L.ntiles = tiles;
     B.L.nvol = nv;
+    B.L.vol0 = B.hvol[0];
+    B.L.coef0 = B.hcoef[0];
     B.L.vol = (const VolDesc*)(m + o_vol);
     B.L.tile_vol = (const int*)(m + o_tile);
     B.L.coef = (const Coef<typename Batch<T, A>::C>*)(m + o_coef);
     B.L.st = (VolState<A>*)(m + o_st);
+    B.L.st_out = B.L.st;
+    B.L.st2 = (VolState<A>*)(m + o_st2);
+    B.L.slot = 0;
     B.L.part = (double*)(m + o_part);
     B.coef64 = (Coef<double>*)(m + o_coef64);
     B.plane_vol = (int*)(m + o_pvol);
@@ -829,7 +836,11 @@ static int solve_plain(fast_ctx* ctx, std::vector<Job*>& jobs, Shape shape, int 
     for (auto* j : jobs) maxit = std::max(maxit, j->prm.max_iter);
     const int chunk = ctx->chunk;
     const long max_chunks = 3 * (maxit / chunk + 2) + 16;
+    int most = 0;
+    for (const VolDesc& d : B.hvol) most = std::max(most, d.ntiles);
+    const bool fold = most <= (sizeof(T) == 8 ? kFoldMaxTilesF64 : kFoldMaxTilesF32);
     auto round = [&]() -> hipError_t {
+        if (fold) return Passes<T, A>::round_folded(B.L, solver, chunk, s);
         for (int i = 0; i < chunk; ++i) {
             hipError_t e2 = (solver == FAST_BICGSTAB) ? Passes<T, A>::bicg_iter(B.L, s) : Passes<T, A>::cg_iter(B.L, s);
             if (e2 != hipSuccess) return e2;

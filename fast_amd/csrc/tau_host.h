@@ -24,6 +24,13 @@ constexpr size_t kMaxSolveVoxels = ((size_t)1 << 29) - 1;
 // Red-black batches launch only the tiles of unfinished volumes once those are at most half
 // of a launch of at least this many tiles.
 constexpr int kRbCompactMin = 512;
+// FP64 and FP32 solves whose volumes have at most this many tiles run each finalize in the next
+// pass's blocks instead of a launch.  Every block of a volume then reads all its partials, and the
+// passes take 8-40 registers more.  MI355X, an iteration of CG / BiCGSTAB with and without: FP64
+// 64^3 (256 tiles) 18.2 / 29.0 and 21.2 / 33.1 us, 100^3 (1000 tiles) 34.9 / 57.3 and 36.5 / 60.1,
+// 256^3 (256) 226 / 428 and 231 / 435; FP32 64^3 16.4 and 18.8, 256^3 (768 tiles, three blocks per CU
+// with 58 registers) 141 and 122.
+constexpr int kFoldMaxTilesF64 = 1100, kFoldMaxTilesF32 = 512;
 // A one-volume red-black launch set of at most this many tiles has its U blocks reduce the
 // Q pass's partials into alpha themselves instead of a finalize launch: the blocks then fit
 // about one dispatch round, so the reduction at their start costs less than the launch it

@@ -115,9 +115,14 @@ struct Launch {
     const int* tile_vol;      // device: tile -> volume
     const Coef<C>* coef;      // device: per volume, in the arithmetic type
     VolState<A>* st;          // device: per volume
+    VolState<A>* st_out;      // where finalizes store the state (= st except in folded rounds)
+    VolState<A>* st2;         // second state buffer of folded rounds
+    int slot;                 // partial-sum slot this pass writes (0; folded rounds alternate 4 and 0)
     double* part;             // device: ntiles * 8 partial sums ((hi, lo) pairs)
     C* tab;                   // device: per volume, kTabEntries diagonals then as many inverses
     VecSet vs;
+    VolDesc vol0;             // the first volume's descriptor and coefficients: what a launch over one
+    Coef<C> coef0;            // volume reads
 };
 
 // Diagonal tables: entry (code | box_x << 7) holds the diagonal of a row with stencil code
@@ -149,6 +154,9 @@ struct Passes {
     static hipError_t cg_iter(const Launch<T, A>&, hipStream_t);
     // Same, recording ev[2k] / ev[2k+1] around stencil pass k (k = 0, 1).
     static hipError_t cg_iter_timed(const Launch<T, A>&, hipStream_t, hipEvent_t* ev);
+    // `iters` iterations with the finalizes inside the next pass (T = A only): one launch per pass
+    // and one per round, where cg_iter and bicg_iter take two per pass.  Same results bit for bit.
+    static hipError_t round_folded(const Launch<T, A>&, int solver, int iters, hipStream_t);
     // Stencil kernel of pass k alone (k = 0, 1 for CG; 0, 1, 2 for BiCGSTAB), no finalize
     // (timing: the volumes' scalars and statuses stay as they are).
     static hipError_t pass_only(const Launch<T, A>&, int solver, int k, hipStream_t);

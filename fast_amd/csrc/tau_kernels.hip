@@ -450,8 +450,10 @@ struct PassOps<T, A, K_CG2> {
 // ahead (compute), and the current plane plus a one-voxel halo is staged in a
 // double-buffered LDS plane; the planes below and above stay in registers.
 // ---------------------------------------------------------------------------------------
-template <class U, class Ops, class Ctx, class Acc, int NPA, int TX, int TY>
-__device__ __forceinline__ void march(const Ctx& pc, const VolDesc& vd, int lt, U* lds, Acc (&acc)[NPA]) {
+// ready() runs once the first planes' loads are in flight and fills in the scalars of `pc` that
+// compute() needs; false ends the march.
+template <class U, class Ops, class Ctx, class Acc, int NPA, int TX, int TY, class Ready>
+__device__ __forceinline__ void march(Ctx& pc, const VolDesc& vd, int lt, U* lds, Acc (&acc)[NPA], Ready ready) {
     using R = typename Ops::R;
     constexpr int W = TX + 2;
     constexpr int PL = (TY + 2) * W;
@@ -510,14 +512,20 @@ __device__ __forceinline__ void march(const Ctx& pc, const VolDesc& vd, int lt, 
     // by that many planes, so a load in flight is never copied; a copy would wait for it).
     constexpr int NB = kPrefetch + 1;
     R rc[NB], rh[NB];
-    if (z0 > 0)
-        u_prev = Ops::compute(pc, Ops::fetch(pc, clin + plane * (z0 - 1), false), bxz(cbxy, z0 - 1), kc(x, y, z0 - 1)).u;
-    c_cur = Ops::compute(pc, Ops::fetch(pc, clin + plane * z0, true), bxz(cbxy, z0), kc(x, y, z0));
-    if (hwave) h_cur = Ops::compute(pc, Ops::fetch(pc, hlin + plane * z0, false), bxz(hbxy, z0), kc(hx, hy, z0)).u;
+    {
+        R r_prev{}, r_cur, r_halo{};
+        if (z0 > 0) r_prev = Ops::fetch(pc, clin + plane * (z0 - 1), false);
+        r_cur = Ops::fetch(pc, clin + plane * z0, true);
+        if (hwave) r_halo = Ops::fetch(pc, hlin + plane * z0, false);
 #pragma unroll
-    for (int j = 0; j < kPrefetch; ++j) {
-        rc[j] = Ops::fetch(pc, clin + plane * clampz(z0 + 1 + j), true);
-        if (hwave) rh[j] = Ops::fetch(pc, hlin + plane * clampz(z0 + 1 + j), false);
+        for (int j = 0; j < kPrefetch; ++j) {
+            rc[j] = Ops::fetch(pc, clin + plane * clampz(z0 + 1 + j), true);
+            if (hwave) rh[j] = Ops::fetch(pc, hlin + plane * clampz(z0 + 1 + j), false);
+        }
+        if (!ready()) return;
+        if (z0 > 0) u_prev = Ops::compute(pc, r_prev, bxz(cbxy, z0 - 1), kc(x, y, z0 - 1)).u;
+        c_cur = Ops::compute(pc, r_cur, bxz(cbxy, z0), kc(x, y, z0));
+        if (hwave) h_cur = Ops::compute(pc, r_halo, bxz(hbxy, z0), kc(hx, hy, z0)).u;
     }
 
     // One plane z: `rc_in` / `rh_in` hold the loads of plane z+1; the loads of plane
@@ -565,7 +573,20 @@ __device__ __forceinline__ void load_tables(const C* src, C* dst, FacePair<C>* f
     __syncthreads();
 }
 
-template <class T, class A, int TX, int TY, int KIND>
+// Number of sums a finalize reads.
+__host__ __device__ constexpr int np_of(int fin) {
+    return fin == F_INIT_CG ? 3 : (fin == F_INIT_BICG || fin == F_BICG2 || fin == F_BICG3 || fin == F_CG2) ? 2 : 1;
+}
+
+// FOLD: the finalize of the previous pass (FinKind), run here instead of in a launch of its own.
+// Every block of a volume reduces that pass's partials and updates a copy of the volume's
+// scalars in LDS while its first planes load: a double-double sum rounds to the same value in
+// any order, so all blocks and k_fin agree to the last bit.  The block of the first tile stores the
+// state to the other of two buffers (blocks that start later still read the old one), and the
+// passes write their partials to alternating slots for the same reason.
+// A finalize launch costs 3.5-4.5 us and a gap on MI355X, the reduction by one wave about 1 us of a
+// block's start.
+template <class T, class A, int TX, int TY, int KIND, int FOLD = -1>
 __global__ __launch_bounds__(TX* TY) void k_stencil(Launch<T, A> L, const T* xin, T* yout) {
     using Ops = PassOps<T, A, KIND>;
     constexpr int NP = Ops::NP;
@@ -577,14 +598,32 @@ __global__ __launch_bounds__(TX* TY) void k_stencil(Launch<T, A> L, const T* xin
 
     const int tile = xcd_remap(blockIdx.x, gridDim.x);
     if (tile >= L.ntiles) return;
-    const int v = L.tile_vol[tile];
-    const VolDesc& vd = L.vol[v];
+    // One volume: its descriptor and coefficients come with the kernel's arguments, so the first
+    // vector loads wait for one dependent load (the state) instead of three.
+    const bool solo = L.nvol == 1;
+    const int v = solo ? 0 : L.tile_vol[tile];
+    VolDesc vd;
+    if (solo)
+        vd = L.vol0;
+    else
+        vd = L.vol[v];
     const VolState<A>* st = L.st + v;
-    if (KIND != K_APPLY && KIND != K_RESTART && st->status != ST_RUNNING) return;
+    __shared__ VolState<A> sst;
+    constexpr int SW = sizeof(VolState<A>) / 4;
+    static_assert(SW <= 256 && sizeof(VolState<A>) % 4 == 0, "one word per thread");
+    const unsigned* st_w = reinterpret_cast<const unsigned*>(st);
+    unsigned* out_w = reinterpret_cast<unsigned*>(L.st_out + v);
+    if (KIND != K_APPLY && KIND != K_RESTART && st->status != ST_RUNNING) {
+        if (FOLD >= 0 && tile == vd.tile_base && (int)threadIdx.x < SW) out_w[threadIdx.x] = st_w[threadIdx.x];
+        return;
+    }
     if (KIND == K_RESTART && st->status != ST_RESTART) return;
 
     PassCtx<T, A> pc;
-    pc.c = L.coef[v];
+    if (solo)
+        pc.c = L.coef0;
+    else
+        pc.c = L.coef[v];
     pc.tab = tab;
     pc.ftab = ftab;
     pc.primary = vd.primary;
@@ -597,7 +636,8 @@ __global__ __launch_bounds__(TX* TY) void k_stencil(Launch<T, A> L, const T* xin
     pc.code = vd.code;
     {
         // per-volume base pointers: element offsets below are within the volume
-        const bool odd = (st->phase & 1) != 0;
+        const int ended = (FOLD == F_CG2 || FOLD == F_BICG3) ? 1 : 0;   // that finalize advances the phase
+        const bool odd = ((st->phase + ended) & 1) != 0;
         const long long o = vd.off;
         pc.x = (T*)L.vs.x + o;
         pc.r = (T*)L.vs.r + o;
@@ -617,13 +657,40 @@ __global__ __launch_bounds__(TX* TY) void k_stencil(Launch<T, A> L, const T* xin
             pc.s = yout + o;
         }
     }
-    load_tables<C, TX * TY>(L.tab + (long long)v * 2 * kTabEntries, tab, ftab, pc.c);
     using Acc = typename AccOf<T, A>::type;
     Acc acc[NPA];
 #pragma unroll
     for (int k = 0; k < NPA; ++k) acc[k].init();
-    march<C, Ops, PassCtx<T, A>, Acc, NPA, TX, TY>(pc, vd, tile - vd.tile_base, lds, acc);
-    if constexpr (NP > 0) block_reduce_store<Acc, NP, TX * TY>(acc, L.part + (long long)tile * kPart);
+    bool go = true;
+    auto ready = [&]() {
+        load_tables<C, TX * TY>(L.tab + (long long)v * 2 * kTabEntries, tab, ftab, pc.c);
+        if constexpr (FOLD >= 0) {
+            constexpr int NPF = np_of(FOLD);
+            // state and sums by the first wave, in order: no barrier before the update
+            if (threadIdx.x < 64)
+                for (int i = (int)threadIdx.x; i < SW; i += 64) reinterpret_cast<unsigned*>(&sst)[i] = st_w[i];
+            double tot[NPF];
+            reduce_volume_wave<NPF>(L.part + (L.slot ^ 4), vd.tile_base, vd.ntiles, tot);
+            if (threadIdx.x == 0) {
+                A ta[3] = {A(0), A(0), A(0)};
+#pragma unroll
+                for (int k = 0; k < NPF; ++k) ta[k] = A(tot[k]);
+                fin_update<A, FOLD>(&sst, ta);
+            }
+            __syncthreads();
+            if (tile == vd.tile_base && (int)threadIdx.x < SW)
+                out_w[threadIdx.x] = reinterpret_cast<const unsigned*>(&sst)[threadIdx.x];
+            pc.first = sst.first;
+            pc.alpha = C(sst.alpha);
+            pc.beta = C(sst.beta);
+            pc.omega = C(sst.omega);
+            go = sst.status == ST_RUNNING;
+        }
+        return go;
+    };
+    march<C, Ops, PassCtx<T, A>, Acc, NPA, TX, TY>(pc, vd, tile - vd.tile_base, lds, acc, ready);
+    if (FOLD >= 0 && !go) return;
+    if constexpr (NP > 0) block_reduce_store<Acc, NP, TX * TY>(acc, L.part + (long long)tile * kPart + L.slot);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -657,11 +724,6 @@ __global__ __launch_bounds__(TX* TY) void k_mixupd(Launch<float, double> L) {
     }
 }
 
-// partial sums each finalize reads
-__host__ __device__ constexpr int np_of(int fin) {
-    return fin == F_INIT_CG ? 3 : (fin == F_INIT_BICG || fin == F_BICG2 || fin == F_BICG3 || fin == F_CG2) ? 2 : 1;
-}
-
 // One block per volume: reduce the volume's tile partials of the pass just run (fixed order)
 // and update its scalars.
 template <class T, class A, int KIND>
@@ -670,6 +732,13 @@ __global__ __launch_bounds__(kFinThreads) void k_fin(Launch<T, A> L) {
     const int v = blockIdx.x;
     if (v >= L.nvol) return;
     VolState<A>* s = L.st + v;
+    if (L.st_out != L.st) {   // end of a folded round: the state moves back to its first buffer
+        constexpr int SW = sizeof(VolState<A>) / 4;
+        if ((int)threadIdx.x < SW)
+            reinterpret_cast<unsigned*>(L.st_out + v)[threadIdx.x] = reinterpret_cast<const unsigned*>(s)[threadIdx.x];
+        s = L.st_out + v;
+        __syncthreads();
+    }
     const int status = s->status;
     if (KIND == F_RESTART) {
         if (status != ST_RESTART) return;
@@ -678,7 +747,7 @@ __global__ __launch_bounds__(kFinThreads) void k_fin(Launch<T, A> L) {
     }
     const VolDesc& vd = L.vol[v];
     double tot[NP];
-    reduce_volume<NP, kFinThreads>(L.part, vd.tile_base, vd.ntiles, tot);
+    reduce_volume<NP, kFinThreads>(L.part + L.slot, vd.tile_base, vd.ntiles, tot);
     if (threadIdx.x == 0) {
         A ta[3] = {A(0), A(0), A(0)};
 #pragma unroll
@@ -716,6 +785,52 @@ hipError_t launch_iter_cg(const Launch<T, A>& L, hipStream_t s, hipEvent_t* ev =
     hipLaunchKernelGGL((k_stencil<T, A, TX, TY, K_CG2>), g, b, 0, s, L, (const T*)nullptr, (T*)nullptr);
     if (ev) (void)hipEventRecord(ev[3], s);
     hipLaunchKernelGGL((k_fin<T, A, F_CG2>), gf, bf, 0, s, L);
+    return hipGetLastError();
+}
+
+// A polling round of `iters` iterations whose passes run the previous pass's finalize themselves;
+// the first pass starts from the state as k_fin left it, the last finalize is a launch.
+template <class T, class A, int TX, int TY>
+hipError_t launch_round(const Launch<T, A>& L0, int solver, int iters, hipStream_t s) {
+    const dim3 g(L0.ntiles), b(TX * TY), gf(L0.nvol), bf(kFinThreads);
+    const T* n0 = nullptr;
+    T* n1 = nullptr;
+    Launch<T, A> L = L0;
+    VolState<A>* buf[2] = {L0.st, L0.st2};
+    int cur = 0;
+    bool folded = false;   // a previous pass of this round is to be finalized
+    auto at = [&](bool fold) {
+        L.st = buf[cur];
+        L.st_out = buf[cur ^ 1];
+        if (fold) cur ^= 1;
+        L.slot ^= 4;
+        folded = true;
+    };
+#define FT_PASS(KIND, PREV)                                                                              \
+    if (folded) {                                                                                        \
+        at(true);                                                                                        \
+        hipLaunchKernelGGL((k_stencil<T, A, TX, TY, KIND, PREV>), g, b, 0, s, L, n0, n1);                \
+    } else {                                                                                             \
+        at(false);                                                                                       \
+        hipLaunchKernelGGL((k_stencil<T, A, TX, TY, KIND>), g, b, 0, s, L, n0, n1);                      \
+    }
+    for (int i = 0; i < iters; ++i) {
+        if (solver == 1) {
+            FT_PASS(K_CG1, F_CG2)
+            FT_PASS(K_CG2, F_CG1)
+        } else {
+            FT_PASS(K_BICG1, F_BICG3)
+            FT_PASS(K_BICG2, F_BICG1)
+            FT_PASS(K_BICG3, F_BICG2)
+        }
+    }
+#undef FT_PASS
+    L.st = buf[cur];
+    L.st_out = L0.st;
+    if (solver == 1)
+        hipLaunchKernelGGL((k_fin<T, A, F_CG2>), gf, bf, 0, s, L);
+    else
+        hipLaunchKernelGGL((k_fin<T, A, F_BICG3>), gf, bf, 0, s, L);
     return hipGetLastError();
 }
 
@@ -890,6 +1005,16 @@ hipError_t Passes<T, A>::cg_iter_timed(const Launch<T, A>& L, hipStream_t s, hip
 }
 
 template <class T, class A>
+hipError_t Passes<T, A>::round_folded(const Launch<T, A>& L, int solver, int iters, hipStream_t s) {
+    if constexpr (sizeof(T) == sizeof(A)) {
+#define FT_CALL(TXV, TYV) return launch_round<T, A, TXV, TYV>(L, solver, iters, s);
+        FT_SHAPES(FT_TRY)
+#undef FT_CALL
+    }
+    return hipErrorInvalidValue;
+}
+
+template <class T, class A>
 hipError_t Passes<T, A>::pass_only(const Launch<T, A>& L, int solver, int k, hipStream_t s) {
 #define FT_CALL(TXV, TYV)                                                                                  \
     {                                                                                                      \
@@ -1028,7 +1153,7 @@ __global__ __launch_bounds__(TX* TY) void k_mixres(Launch<float, double> L, cons
     AccDD acc[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) acc[k].init();
-    march<double, MixOps, MixCtx, AccDD, 4, TX, TY>(pc, vd, tile - vd.tile_base, lds, acc);
+    march<double, MixOps, MixCtx, AccDD, 4, TX, TY>(pc, vd, tile - vd.tile_base, lds, acc, [] { return true; });
     block_reduce_store<AccDD, 4, TX * TY>(acc, L.part + (long long)tile * kPart);
 }
 
