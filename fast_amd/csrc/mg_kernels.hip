@@ -41,6 +41,10 @@ __device__ __forceinline__ float mg_sum(const FacePair<float>* ftab, int code, c
     return acc;
 }
 
+__device__ __forceinline__ MgFine mg_fine(const MgDesc& d) {
+    return MgFine{d.tiles_x, d.tiles_y, d.tz, d.part_base, d.lev[0].nx, d.lev[0].ny, d.mem + d.lev[0].off};
+}
+
 // Fine level.  Geometry, rings and LDS planes as in k_rb_yq (columns that march z, p planes
 // double-buffered, Y planes in a ring, one barrier per plane), in FP32:
 //   pre:  u = x1; Y = (1/|D_b|) A_br u; G = A_rb Y on the red voxels, summed over the four red
@@ -60,18 +64,24 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
     static_assert(kRbTX == 64 && NPO <= 3 * 64, "one p-only point per lane of waves TY .. TY+2");
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= M.ntiles) return;
-    const int2 tl = M.tiles[slot];
-    const int v = tl.x, lt = tl.y;
+    int2 tl{0, slot};
+    if (!L.solo) tl = M.tiles[slot];
+    const int v = uniform(tl.x), lt = uniform(tl.y);
     const VolState<double>* vs = L.st + v;
     if (vs->status != ST_RUNNING || !vs->mg) return;
-    const RbDesc d = L.vol[v];
-    const MgDesc& md = M.vol[v];
+    const RbDesc d = rb_desc(L, v);
+    MgFine md;
+    if (L.solo)
+        md = mg_fine(M.vol0);
+    else
+        md = mg_fine(M.vol[v]);
+    md = uniform(md);
     __shared__ float tab[kTabEntries];
     __shared__ FacePair<float> ftab[8];
     __shared__ float pbuf[2][PW * PH + 1];
     __shared__ float ybuf[R][YW * YH + 1];
     __shared__ float rows[2][TY / 2][kRbTX];
-    const Coef<double> c = L.coef[v];
+    const Coef<double> c = rb_coef(L, v);
     const Coef<float> cf{(float)c.ci0, (float)c.ci1, (float)c.ci2, (float)c.cb0, (float)c.cb1, 0.0f, 0.0f, 0.0f, 0.0f};
     for (int i = (int)threadIdx.x; i < kTabEntries; i += NT) tab[i] = M.tab[(long long)v * kTabEntries + i];
     if (threadIdx.x < 8) ftab[threadIdx.x] = face_pair(cf, (int)threadIdx.x);
@@ -86,8 +96,8 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
     float* Z = L.p[odd ? 0 : 1] + d.off_c;
     const unsigned* code_r4 = reinterpret_cast<const unsigned*>(d.code_c[0]);
     const unsigned* code_b4 = reinterpret_cast<const unsigned*>(d.code_c[1]);
-    const int cnx = md.lev[0].nx, cny = md.lev[0].ny;
-    float* G1 = md.mem + md.lev[0].off;
+    const int cnx = md.cnx, cny = md.cny;
+    float* G1 = md.g1;
     const int tid = (int)threadIdx.x, w = tid >> 6, lane = tid & 63;
     // this thread's column (slot kc, row yc)
     const bool own = w < TY;
@@ -152,8 +162,11 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
     AccDD acc[1];
     acc[0].init();
     const int t0 = z0 - 1;
-    float pr[R], po[R], er[R], eo[R], rr[R];
-    unsigned cb[R], cr[R];
+    // Rings: u, the p-only point and the black code of planes t-1 .. t+2; the red code and r of planes
+    // t-1 and t (issued first in a step, so waiting for them leaves the later loads in flight); e of
+    // two plane pairs (t0 is odd, so a plane's pair is a constant of its ring index).
+    float pr[R], po[R], er[2], eo[2], rr[2];
+    unsigned cb[R], cr[2];
     // u of plane zz from its loads: the correction is added on the red voxels of the box
     auto finish_col = [&](int zz, float x, float e) {
         const bool ok = (((~sb0 ^ zz) & 1) ? ok1 : ok0) && (unsigned)zz < (unsigned)d.nz;
@@ -164,49 +177,45 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
         return ok ? x + e : x;
     };
     pr[R - 1] = ld(X1 + plane(t0 - 1), cel);
-    if (POST) er[R - 1] = ld(G1 + eplane(t0 - 1), ecol);
-    cr[R - 1] = 0;
-    rr[R - 1] = 0.0f;
+    if (POST) {
+        er[1] = ld(G1 + eplane(t0), ecol);   // planes t0 - 1 and t0
+        eo[1] = ld(G1 + eplane(t0), epel);
+        er[0] = ld(G1 + eplane(t0 + 1), ecol);
+        eo[0] = ld(G1 + eplane(t0 + 1), epel);
+    }
+    cr[1] = 0;   // q(t0 - 1) is never formed
+    rr[1] = 0.0f;
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i) {
         const unsigned o = plane(t0 + i);
         pr[i] = ld(X1 + o, cel);
         po[i] = ld(X1 + o, pel);
-        if (POST) {
-            er[i] = ld(G1 + eplane(t0 + i), ecol);
-            eo[i] = ld(G1 + eplane(t0 + i), epel);
-        }
         cb[i] = ld(code_b4 + (o >> 2), cel4);
-        if (i < AHEAD - 1) {
-            cr[i] = ld(code_r4 + (o >> 2), cel4);
-            if (POST) rr[i] = ld(Rr + o, cel);
-        }
     }
     if (POST) {
-        pr[R - 1] = finish_col(t0 - 1, pr[R - 1], er[R - 1]);
-        pr[0] = finish_col(t0, pr[0], er[0]);
+        pr[R - 1] = finish_col(t0 - 1, pr[R - 1], er[1]);
+        pr[0] = finish_col(t0, pr[0], er[1]);
     }
     float hold = 0.0f;   // pre: G of the pair's first plane
     auto step = [&](auto J, int t) {
         constexpr int j = decltype(J)::value;
         constexpr int jm = (j + R - 1) % R, jn = (j + 1) % R;
         {
-            const unsigned o = plane(t + AHEAD), oq = plane(t + AHEAD - 1);
+            const unsigned oq = plane(t), o = plane(t + AHEAD);
+            cr[j & 1] = ld(code_r4 + (oq >> 2), cel4);
+            if (POST) rr[j & 1] = ld(Rr + oq, cel);
             pr[(j + AHEAD) % R] = ld(X1 + o, cel);
             po[(j + AHEAD) % R] = ld(X1 + o, pel);
             cb[(j + AHEAD) % R] = ld(code_b4 + (o >> 2), cel4);
-            cr[(j + AHEAD - 1) % R] = ld(code_r4 + (oq >> 2), cel4);
-            if (POST) {
-                const unsigned eo_ = eplane(t + AHEAD);
-                er[(j + AHEAD) % R] = ld(G1 + eo_, ecol);
-                eo[(j + AHEAD) % R] = ld(G1 + eo_, epel);
-                rr[(j + AHEAD - 1) % R] = ld(Rr + oq, cel);
+            if (POST && (j & 1)) {   // plane t + 2 opens a pair
+                er[((j + 1) >> 1) & 1] = ld(G1 + eplane(t + AHEAD), ecol);
+                eo[((j + 1) >> 1) & 1] = ld(G1 + eplane(t + AHEAD), epel);
             }
         }
-        if (POST) pr[jn] = finish_col(t + 1, pr[jn], er[jn]);
+        if (POST) pr[jn] = finish_col(t + 1, pr[jn], er[(j >> 1) & 1]);
         float* pb = pbuf[t & 1];
         pb[pdst] = pr[j];
-        pb[podst] = POST ? finish_po(t, po[j], eo[j]) : po[j];
+        pb[podst] = POST ? finish_po(t, po[j], eo[((j + 3) >> 1) & 1]) : po[j];
         __syncthreads();
         const int s = sb0 ^ (t & 1);
         const float* pl = pb + pdst;
@@ -222,12 +231,12 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
         if (red) {
             const float* yl = ybuf[jm] + ypos;
             const float o[6] = {ybuf[(j + R - 2) % R][ypos], yl[-YW], yl[s - 1], yl[s], yl[YW], yt};
-            const int code_q = (int)((cr[jm] >> csh) & 0xffu);
+            const int code_q = (int)((cr[(j + 1) & 1] >> csh) & 0xffu);
             g = mg_sum(ftab, code_q, o);
             if (POST) {
-                const float zv = (g - rr[jm]) * inv(code_q, s, yc, tq, tq == 0 || tq == d.nz - 1);
+                const float zv = (g - rr[(j + 1) & 1]) * inv(code_q, s, yc, tq, tq == 0 || tq == d.nz - 1);
                 st(Z + d.pp * (unsigned)(tq + 1), cel, zv);
-                acc[0].add(rr[jm], zv);
+                acc[0].add(rr[(j + 1) & 1], zv);
             }
         }
         if (!POST) {
@@ -265,21 +274,20 @@ struct MgLev {
     float* gc;                       // next level's g
 };
 
-__device__ __forceinline__ MgLev mg_lev(const MgDesc& d, int l) {
+__device__ __forceinline__ MgLev mg_lev(const MgLevel& a, const MgLevel& c, float* mem) {
     MgLev r;
-    const MgLevel& a = d.lev[l];
     r.nx = a.nx;
     r.ny = a.ny;
     r.nz = a.nz;
     r.cx = half_up(a.nx);
     r.cy = half_up(a.ny);
-    r.g = d.mem + a.off;
+    r.g = mem + a.off;
     r.t = r.g + a.n;
     r.fx = r.t + a.n;
     r.fy = r.fx + a.n;
     r.fz = r.fy + a.n;
     r.iv = r.fz + a.n;
-    r.gc = d.mem + d.lev[l + 1].off;
+    r.gc = mem + c.off;
     return r;
 }
 
@@ -332,6 +340,15 @@ __device__ __forceinline__ float mg_dot(const float (&f)[6], const float (&u)[6]
     return fmaf(f[5], u[5], a);
 }
 
+struct MgLevelArgs {
+    const VolState<double>* st;
+    const MgDesc* vol;
+    const int2* blocks;
+    int nblk, lev;
+    float* mem;         // solo launches: the volume's level storage, this level and the next
+    MgLevel la, lc;
+};
+
 enum MgStep : int { MG_PRE_BLACK = 0, MG_RESTRICT, MG_POST_BLACK, MG_POST_RED };
 
 // Half sweeps of one level:
@@ -340,15 +357,23 @@ enum MgStep : int { MG_PRE_BLACK = 0, MG_RESTRICT, MG_POST_BLACK, MG_POST_RED };
 //   post black: g = (g + sum c (g_r iv_r + e)) iv on black cells, e the next level's solution
 //   post red:   g = (g + sum c g_b) iv on red cells (g is then the level's solution)
 template <int STEP>
-__global__ __launch_bounds__(kMgThreads) void k_mg_level(RbLaunch L, const MgDesc* vol, const int2* blocks, int nblk, int lev) {
+__global__ __launch_bounds__(kMgThreads) void k_mg_level(MgLevelArgs A) {
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
-    if (slot >= nblk) return;
-    const int2 b = blocks[slot];
-    if (L.st[b.x].status != ST_RUNNING || !L.st[b.x].mg) return;
-    const MgDesc& d = vol[b.x];
-    const MgLev l = mg_lev(d, lev);
+    if (slot >= A.nblk) return;
+    int2 b{0, slot};
+    MgLevel la = A.la, lc = A.lc;
+    float* mem = A.mem;
+    if (!mem) {   // not a solo launch
+        b = A.blocks[slot];
+        la = A.vol[b.x].lev[A.lev];
+        lc = A.vol[b.x].lev[A.lev + 1];
+        mem = A.vol[b.x].mem;
+    }
+    if (A.st[b.x].status != ST_RUNNING || !A.st[b.x].mg) return;
+    b = uniform(b);
+    const MgLev l = mg_lev(uniform(la), uniform(lc), uniform(mem));
     const unsigned id = (unsigned)b.y * kMgThreads + threadIdx.x;
-    const unsigned C = id >> 2, nc = (unsigned)d.lev[lev + 1].n;
+    const unsigned C = id >> 2, nc = (unsigned)lc.n;
     constexpr int colour = (STEP == MG_PRE_BLACK || STEP == MG_POST_BLACK) ? 1 : 0;
     MgCell c = mg_cell(l.nx, l.ny, l.nz, l.cx, l.cy, C < nc ? C : 0u, (int)(id & 3u), colour);
     c.ok = c.ok && C < nc;
@@ -401,45 +426,74 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_level(RbLaunch L, const MgDes
 }
 
 // The levels from `bottom` on, one block per volume, in LDS: one V-cycle with two sweeps before
-// and after each correction, down to a level of one cell, whose equation is solved.  t holds the
-// iterate u.  (Two sweeps here save 3-15% of the CG's iterations at no further launches.  A second
-// V-cycle on the first one's residual saves as many, but 2 B - B A B is indefinite where the
-// cycle overcorrects, as in long clogged volumes.)
+// and after each correction; the last level (at most 64 cells) is solved with its inverse.  t
+// holds the iterate u.  (Two sweeps here save 3-15% of the CG's iterations at no further launches.
+// A second V-cycle on the first one's residual saves as many, but 2 B - B A B is indefinite
+// where the cycle overcorrects, as in long clogged volumes.)
+// Bound by the chain of phases (a phase is one half sweep and a barrier, about 0.4 us): 16^3 cells
+// took 26 us with levels down to one cell, integer divisions and level data read from memory in
+// every phase; now eight phases a level, two levels and one product.
 constexpr int kMgBottomThreads = 1024;
 
 struct LdsLev {
     int nx, ny, nz, cx, cy, n, nc;
+    unsigned mx, my;   // ceil(2^32 / cx), ceil(2^32 / cy): exact quotients for the cells kept here
     float *g, *t, *fx, *fy, *fz, *iv, *gc, *tc;
 };
 
+__device__ __forceinline__ MgCell lds_cell(const LdsLev& q, unsigned C, int j, int colour) {
+    const unsigned row = q.cx == 1 ? C : __umulhi(C, q.mx);
+    const int K = (int)(C - row * (unsigned)q.cx);
+    const unsigned Zu = q.cy == 1 ? row : __umulhi(row, q.my);
+    const int Z = (int)Zu, Y = (int)(row - Zu * (unsigned)q.cy);
+    MgCell c;
+    c.y = 2 * Y + (j & 1);
+    c.z = 2 * Z + (j >> 1);
+    c.x = 2 * K + ((colour + c.y + c.z) & 1);
+    c.ok = c.x < q.nx && c.y < q.ny && c.z < q.nz;
+    c.i = (unsigned)c.x + (unsigned)q.nx * ((unsigned)c.y + (unsigned)q.ny * (unsigned)c.z);
+    return c;
+}
+
 __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLaunch M) {
     __shared__ float sm[kMgArrays][kMgBottomCells];
-    const int v = M.vols[blockIdx.x];
+    __shared__ MgLevel sl[kMgLevels];
+    const int v = L.solo ? 0 : M.vols[blockIdx.x];
     if (L.st[v].status != ST_RUNNING || !L.st[v].mg) return;
     const MgDesc& d = M.vol[v];
     const int tid = (int)threadIdx.x;
     const int b = d.bottom, last = d.nlev - 1;
+    float* mem = d.mem;
+    // row tid / 16 of the last level's inverse (64 x 64, padded with zeros), columns 4 (tid % 16) ..
+    const float4 inv = reinterpret_cast<const float4*>(mem + d.inv_off)[tid];
+    if (tid >= b && tid <= last) sl[tid] = d.lev[tid];
+    __syncthreads();
     // cells of a level start at its offset from the bottom level (all arrays alike)
-    auto lds_off = [&](int l) { return (int)((d.lev[l].off - d.lev[b].off) / kMgArrays); };
+    const unsigned off_b = sl[b].off;
+    auto lds_off = [&](int l) { return (int)((sl[l].off - off_b) / kMgArrays); };
     for (int l = b; l <= last; ++l) {
-        const int n = d.lev[l].n, o = lds_off(l);
-        const float* src = d.mem + d.lev[l].off;
+        const int n = sl[l].n, o = lds_off(l);
+        const float* src = mem + sl[l].off;
         for (int i = tid; i < n; i += kMgBottomThreads) {
             if (l == b) sm[0][o + i] = src[i];
+            if (l < last) {
 #pragma unroll
-            for (int a = 2; a < kMgArrays; ++a) sm[a][o + i] = src[(long long)a * n + i];
+                for (int a = 2; a < kMgArrays; ++a) sm[a][o + i] = src[(long long)a * n + i];
+            }
         }
     }
     auto level = [&](int l) {
         LdsLev r;
-        const int o = lds_off(l), oc = l < last ? lds_off(l + 1) : o;
-        r.nx = d.lev[l].nx;
-        r.ny = d.lev[l].ny;
-        r.nz = d.lev[l].nz;
+        const int o = lds_off(l), oc = lds_off(l + 1);
+        r.nx = sl[l].nx;
+        r.ny = sl[l].ny;
+        r.nz = sl[l].nz;
         r.cx = half_up(r.nx);
         r.cy = half_up(r.ny);
-        r.n = d.lev[l].n;
-        r.nc = l < last ? d.lev[l + 1].n : 0;
+        r.mx = 0xFFFFFFFFu / (unsigned)r.cx + 1u;
+        r.my = 0xFFFFFFFFu / (unsigned)r.cy + 1u;
+        r.n = sl[l].n;
+        r.nc = sl[l + 1].n;
         r.g = sm[0] + o;
         r.t = sm[1] + o;
         r.fx = sm[2] + o;
@@ -450,13 +504,12 @@ __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLa
         r.tc = sm[1] + oc;
         return r;
     };
-    // f(cell) for this thread's cells of one colour, then a barrier
+    // f(cell) for this thread's cells of one colour
     auto cells = [&](const LdsLev& q, int colour, auto f) {
         for (int id = tid; id < 4 * q.nc; id += kMgBottomThreads) {
-            const MgCell c = mg_cell(q.nx, q.ny, q.nz, q.cx, q.cy, (unsigned)id >> 2, id & 3, colour);
+            const MgCell c = lds_cell(q, (unsigned)id >> 2, id & 3, colour);
             if (c.ok) f(c);
         }
-        __syncthreads();
     };
     auto sweep = [&](const LdsLev& q, int colour) {
         cells(q, colour, [&](const MgCell& c) {
@@ -467,20 +520,29 @@ __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLa
             for (int k = 0; k < 6; ++k) u[k] = q.t[n[k]];   // a box face's coefficient is 0, t finite
             q.t[c.i] = (q.g[c.i] + mg_dot(f, u)) * q.iv[c.i];
         });
+        __syncthreads();
     };
     __syncthreads();
     for (int l = b; l < last; ++l) {
         const LdsLev q = level(l);
-        for (int i = tid; i < q.n; i += kMgBottomThreads) q.t[i] = q.g[i] * q.iv[i];   // red sweep from zero
+        // red sweep from zero and the black one after it, at once: the red values are g iv
+        cells(q, 0, [&](const MgCell& c) { q.t[c.i] = q.g[c.i] * q.iv[c.i]; });
+        cells(q, 1, [&](const MgCell& c) {
+            float f[6], u[6];
+            unsigned n[6];
+            mg_faces(q, c, f, n);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) u[k] = q.g[n[k]] * q.iv[n[k]];
+            q.t[c.i] = (q.g[c.i] + mg_dot(f, u)) * q.iv[c.i];
+        });
         __syncthreads();
-        sweep(q, 1);
         sweep(q, 0);
         sweep(q, 1);
         for (int i0 = 0; i0 < 4 * q.nc; i0 += kMgBottomThreads) {   // whole waves: lanes are summed
             const int id = i0 + tid;
             float s = 0.0f;
             if (id < 4 * q.nc) {
-                const MgCell c = mg_cell(q.nx, q.ny, q.nz, q.cx, q.cy, (unsigned)id >> 2, id & 3, 0);
+                const MgCell c = lds_cell(q, (unsigned)id >> 2, id & 3, 0);
                 if (c.ok && q.iv[c.i] > 0.0f) {
                     float f[6], u[6];
                     unsigned n[6];
@@ -496,34 +558,57 @@ __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLa
         }
         __syncthreads();
     }
-    if (tid == 0) {
-        const LdsLev q = level(last);
-        q.t[0] = q.g[0] * q.iv[0];
+    {
+        const int n = sl[last].n, o = lds_off(last), c = 4 * (tid & 15);
+        const float* g = sm[0] + o;
+        float s = inv.x * (c < n ? g[c] : 0.0f);
+        s = fmaf(inv.y, c + 1 < n ? g[c + 1] : 0.0f, s);
+        s = fmaf(inv.z, c + 2 < n ? g[c + 2] : 0.0f, s);
+        s = fmaf(inv.w, c + 3 < n ? g[c + 3] : 0.0f, s);
+#pragma unroll
+        for (int k = 1; k < 16; k <<= 1) s += __shfl_xor(s, k, 64);
+        if ((tid & 15) == 0 && (tid >> 4) < n) sm[1][o + (tid >> 4)] = s;
     }
     __syncthreads();
     for (int l = last - 1; l >= b; --l) {
         const LdsLev q = level(l);
-        cells(q, 0, [&](const MgCell& c) { q.t[c.i] += q.tc[(c.x >> 1) + q.cx * ((c.y >> 1) + q.cy * (c.z >> 1))]; });
-        sweep(q, 1);
+        // black sweep on u_r + e (the red sweep after it replaces u_r, so e is never added there)
+        cells(q, 1, [&](const MgCell& c) {
+            float f[6], u[6], e[6];
+            unsigned n[6];
+            mg_faces(q, c, f, n);
+            const int px = q.cx, pxy = q.cx * q.cy;
+            const int cb = (c.y >> 1) * px + (c.z >> 1) * pxy, base = cb + (c.x >> 1);
+            e[0] = q.tc[c.x > 0 ? cb + ((c.x - 1) >> 1) : base];
+            e[1] = q.tc[c.x + 1 < q.nx ? cb + ((c.x + 1) >> 1) : base];
+            e[2] = q.tc[c.y > 0 && !(c.y & 1) ? base - px : base];
+            e[3] = q.tc[c.y + 1 < q.ny && (c.y & 1) ? base + px : base];
+            e[4] = q.tc[c.z > 0 && !(c.z & 1) ? base - pxy : base];
+            e[5] = q.tc[c.z + 1 < q.nz && (c.z & 1) ? base + pxy : base];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) u[k] = f[k] != 0.0f ? q.t[n[k]] + e[k] : 0.0f;   // not t of this cell, being written
+            q.t[c.i] = (q.g[c.i] + mg_dot(f, u)) * q.iv[c.i];
+        });
+        __syncthreads();
         sweep(q, 0);
         sweep(q, 1);
         sweep(q, 0);
     }
-    float* out = d.mem + d.lev[b].off;
-    const LdsLev q = level(b);
-    for (int i = tid; i < q.n; i += kMgBottomThreads) out[i] = q.t[i];
+    const float* u = sm[1];
+    for (int i = tid; i < sl[b].n; i += kMgBottomThreads) mem[off_b + i] = u[i];
 }
 
 // r.z of one preconditioned volume, then beta = r.z / (previous r.z).
 __global__ __launch_bounds__(kFinThreads) void k_mg_fin(RbLaunch L, MgLaunch M) {
-    const int v = M.vols[blockIdx.x];
+    const int v = L.solo ? 0 : M.vols[blockIdx.x];
     VolState<double>* s = L.st + v;
     if (s->status != ST_RUNNING || !s->mg) return;
-    const MgDesc& d = M.vol[v];
+    const int ntiles = L.solo ? M.vol0.ntiles : M.vol[v].ntiles;
+    const int base = L.solo ? M.vol0.part_base : M.vol[v].part_base;
     AccDD sum[1];
     sum[0].init();
-    for (int i = (int)threadIdx.x; i < d.ntiles; i += kFinThreads) {
-        const double* p = M.part + 2 * ((long long)d.part_base + i);
+    for (int i = (int)threadIdx.x; i < ntiles; i += kFinThreads) {
+        const double* p = M.part + 2 * ((long long)base + i);
         sum[0].add2(p[0], p[1]);
     }
     __shared__ double red[2];
@@ -551,86 +636,134 @@ __device__ __forceinline__ float mg_series(float m, float l, bool has_l, float r
     return m > 0.0f ? fmaxf(1.0f / R, kMgFaceMin * m) : 0.0f;
 }
 
-// Coefficients of level l from the stencil codes (l = 0) or from level l - 1: the faces towards
-// x+, y+, z+ and, in t, the cell's half-cell faces on the primary axis.
-__global__ __launch_bounds__(kMgThreads) void k_mg_coef(RbLaunch L, MgLaunch M, int lev) {
+// Coefficients of the first level from the stencil codes: the faces towards x+, y+, z+ and, in t, the
+// cell's half-cell faces on the primary axis.  A code holds its voxel's and its neighbours' solid flags,
+// so a cell's own faces and those towards + take its 8 children's codes, and the next cells' inner
+// faces 4 codes each: 20 independent byte loads (256^3: 400 us with a loop over the faces on 512
+// blocks, 43 us so).
+__global__ __launch_bounds__(kMgThreads) void k_mg_coef0(RbLaunch L, MgLaunch M) {
     const int v = M.vols[blockIdx.y];
     const MgDesc& d = M.vol[v];
-    if (lev >= d.nlev) return;
-    const MgLevel& a = d.lev[lev];
+    const MgLevel a = d.lev[0];
     const RbDesc& rb = L.vol[v];
+    const uint8_t* code = rb.code;
     float* g = d.mem + a.off;
     float *t = g + a.n, *fx = t + a.n, *fy = fx + a.n, *fz = fy + a.n;
-    const int fn[3] = {lev ? d.lev[lev - 1].nx : rb.nx, lev ? d.lev[lev - 1].ny : rb.ny, lev ? d.lev[lev - 1].nz : rb.nz};
+    const int fn[3] = {rb.nx, rb.ny, rb.nz};
     const int primary = rb.primary;
     const Coef<double> c = L.coef[v];
-    const float ci[3] = {(float)c.ci0, (float)c.ci1, (float)c.ci2};
-    const float cb[2] = {(float)c.cb0, (float)c.cb1};
-    const float* pf[3] = {nullptr, nullptr, nullptr};
-    const float* pt = nullptr;
-    if (lev) {
-        const MgLevel& p = d.lev[lev - 1];
-        const float* m = d.mem + p.off;
-        pt = m + p.n;
-        pf[0] = pt + p.n;
-        pf[1] = pf[0] + p.n;
-        pf[2] = pf[1] + p.n;
-    }
+    const float c0 = (float)c.ci0, c1 = (float)c.ci1, c2 = (float)c.ci2, b0 = (float)c.cb0, b1 = (float)c.cb1;
     const unsigned st[3] = {1u, (unsigned)fn[0], (unsigned)fn[0] * (unsigned)fn[1]};
-    // face of child fi towards + along axis q (inside the box)
-    auto face = [&](unsigned fi, int q) {
-        if (lev) return pf[q][fi];
-        const int code = rb.code[fi];
-        return ci[((code >> 6) & 1) + ((code >> (2 * q)) & 1)];
-    };
-    // sum of the faces towards + along q of the children at plane k (along q) of the coarse cell I
-    auto sum4 = [&](const int (&I)[3], int q, int k) {
-        const int u = q == 0 ? 1 : 0, w = q == 2 ? 1 : 2;
-        float s = 0.0f;
-        for (int j = 0; j < 4; ++j) {
-            const int a0 = 2 * I[u] + (j & 1), a1 = 2 * I[w] + (j >> 1);
-            if (a0 < fn[u] && a1 < fn[w]) s += face((unsigned)a0 * st[u] + (unsigned)a1 * st[w] + (unsigned)k * st[q], q);
-        }
-        return s;
-    };
+    // face between voxels of solid flags o and n
+    auto face = [&](int o, int n) { return o + n == 0 ? c0 : (o + n == 1 ? c1 : c2); };
     for (unsigned i = blockIdx.x * kMgThreads + threadIdx.x; i < (unsigned)a.n; i += gridDim.x * kMgThreads) {
         const unsigned row = i / (unsigned)a.nx;
         const int I[3] = {(int)(i - row * (unsigned)a.nx), (int)(row % (unsigned)a.ny), (int)(row / (unsigned)a.ny)};
+        const unsigned o = 2u * (unsigned)I[0] + 2u * (unsigned)I[1] * st[1] + 2u * (unsigned)I[2] * st[2];
+        bool two[3], next[3], wide[3];   // two children; a next cell; two children in the next cell
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            two[q] = 2 * I[q] + 1 < fn[q];
+            next[q] = 2 * I[q] + 2 < fn[q];
+            wide[q] = 2 * I[q] + 3 < fn[q];
+        }
+        int ch[8];      // children (bit q of the index: upper along axis q); -1 outside the box
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const bool in = (!(j & 1) || two[0]) && (!(j & 2) || two[1]) && (!(j & 4) || two[2]);
+            const int v8 = code[in ? o + (unsigned)(j & 1) + (unsigned)((j >> 1) & 1) * st[1] + (unsigned)(j >> 2) * st[2] : o];
+            ch[j] = in ? v8 : -1;
+        }
         float s[3], own[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            const int lo = 2 * I[q], nq = fn[q];
-            own[q] = lo + 1 < nq ? sum4(I, q, lo) : 0.0f;
-            s[q] = 0.0f;
-            if (lo + 2 < nq) {
-                const bool wide = lo + 3 < nq;   // the next cell has two children
-                s[q] = mg_series(sum4(I, q, lo + 1), own[q], true, wide ? sum4(I, q, lo + 2) : 0.0f, wide);
+            const int u = q == 0 ? 1 : 0, w = q == 2 ? 1 : 2;
+            float in = 0.0f, m = 0.0f, r = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int lo = ((j & 1) << u) | ((j >> 1) << w), hi = lo | (1 << q);
+                const unsigned nx = o + 2u * st[q] + (unsigned)(j & 1) * st[u] + (unsigned)(j >> 1) * st[w];
+                const int cn = code[next[q] && ch[lo] >= 0 ? nx : o];
+                if (two[q] && ch[lo] >= 0) in += face((ch[lo] >> 6) & 1, (ch[lo] >> (2 * q)) & 1);
+                if (next[q] && ch[hi] >= 0) m += face((ch[hi] >> 6) & 1, (ch[hi] >> (2 * q)) & 1);
+                if (wide[q] && ch[lo] >= 0) r += face((cn >> 6) & 1, (cn >> (2 * q)) & 1);
             }
+            own[q] = in;
+            s[q] = next[q] ? mg_series(m, in, true, r, wide[q]) : 0.0f;
         }
         // half-cell faces at either end of the primary axis
-        const int np = fn[primary], lo = 2 * I[primary];
-        const float inner = primary == 0 ? own[0] : (primary == 1 ? own[1] : own[2]);
         float end[2] = {0.0f, 0.0f};
+        const int Ip = primary == 0 ? I[0] : (primary == 1 ? I[1] : I[2]), np = primary == 0 ? fn[0] : (primary == 1 ? fn[1] : fn[2]);
+#pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int x[3] = {2 * I[0] + (j & 1), 2 * I[1] + ((j >> 1) & 1), 2 * I[2] + (j >> 2)};
-            if (x[0] >= fn[0] || x[1] >= fn[1] || x[2] >= fn[2]) continue;
-            const int k = primary == 0 ? x[0] : (primary == 1 ? x[1] : x[2]);
-            if (k != 0 && k != np - 1) continue;
-            const unsigned fi = (unsigned)x[0] + (unsigned)x[1] * st[1] + (unsigned)x[2] * st[2];
-            if (lev) {
-                end[k == 0 ? 0 : 1] += pt[fi];   // one cell along the axis: both ends together
-            } else {
-                const float h = cb[(rb.code[fi] >> 6) & 1];
-                if (k == 0) end[0] += h;
-                if (k == np - 1) end[1] += h;
-            }
+            if (ch[j] < 0) continue;
+            const int k = 2 * Ip + ((j >> primary) & 1);
+            const float h = (ch[j] >> 6) & 1 ? b1 : b0;
+            if (k == 0) end[0] += h;
+            if (k == np - 1) end[1] += h;
         }
-        const bool two = lo + 1 < np;   // two children along the axis
+        const float inner = primary == 0 ? own[0] : (primary == 1 ? own[1] : own[2]);
+        const bool tp = 2 * Ip + 1 < np;
         g[i] = 0.0f;
         fx[i] = s[0];
         fy[i] = s[1];
         fz[i] = s[2];
-        t[i] = mg_series(end[0], inner, two, 0.0f, false) + mg_series(end[1], inner, two, 0.0f, false);
+        t[i] = mg_series(end[0], inner, tp, 0.0f, false) + mg_series(end[1], inner, tp, 0.0f, false);
+    }
+}
+
+// The same of level `lev` >= 1 from level lev - 1.
+__global__ __launch_bounds__(kMgThreads) void k_mg_coef(RbLaunch L, MgLaunch M, int lev) {
+    const int v = M.vols[blockIdx.y];
+    const MgDesc& d = M.vol[v];
+    if (lev >= d.nlev) return;
+    const MgLevel a = d.lev[lev], p = d.lev[lev - 1];
+    const int primary = L.vol[v].primary;
+    float* g = d.mem + a.off;
+    float *t = g + a.n, *fx = t + a.n, *fy = fx + a.n, *fz = fy + a.n;
+    const int fn[3] = {p.nx, p.ny, p.nz};
+    const float* pt = d.mem + p.off + p.n;
+    const unsigned st[3] = {1u, (unsigned)fn[0], (unsigned)fn[0] * (unsigned)fn[1]};
+    for (unsigned i = blockIdx.x * kMgThreads + threadIdx.x; i < (unsigned)a.n; i += gridDim.x * kMgThreads) {
+        const unsigned row = i / (unsigned)a.nx;
+        const int I[3] = {(int)(i - row * (unsigned)a.nx), (int)(row % (unsigned)a.ny), (int)(row / (unsigned)a.ny)};
+        const unsigned o = 2u * (unsigned)I[0] + 2u * (unsigned)I[1] * st[1] + 2u * (unsigned)I[2] * st[2];
+        float s[3], own[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int u = q == 0 ? 1 : 0, w = q == 2 ? 1 : 2;
+            const float* f = pt + (size_t)(q + 1) * p.n;   // faces towards + along q
+            const bool two = 2 * I[q] + 1 < fn[q], next = 2 * I[q] + 2 < fn[q], wide = 2 * I[q] + 3 < fn[q];
+            float in = 0.0f, m = 0.0f, r = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool ok = 2 * I[u] + (j & 1) < fn[u] && 2 * I[w] + (j >> 1) < fn[w];
+                const unsigned b = o + (ok ? (unsigned)(j & 1) * st[u] + (unsigned)(j >> 1) * st[w] : 0u);
+                const float f0 = f[b], f1 = f[next ? b + st[q] : b], f2 = f[wide ? b + 2u * st[q] : b];
+                in += ok && two ? f0 : 0.0f;
+                m += ok && next ? f1 : 0.0f;
+                r += ok && wide ? f2 : 0.0f;
+            }
+            own[q] = in;
+            s[q] = next ? mg_series(m, in, true, r, wide) : 0.0f;
+        }
+        // half-cell faces at either end of the primary axis (one cell along it: both ends together)
+        const int Ip = primary == 0 ? I[0] : (primary == 1 ? I[1] : I[2]), np = primary == 0 ? fn[0] : (primary == 1 ? fn[1] : fn[2]);
+        float end[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const bool ok = 2 * I[0] + (j & 1) < fn[0] && 2 * I[1] + ((j >> 1) & 1) < fn[1] && 2 * I[2] + (j >> 2) < fn[2];
+            const int k = 2 * Ip + ((j >> primary) & 1);
+            if (!ok || (k != 0 && k != np - 1)) continue;
+            end[k == 0 ? 0 : 1] += pt[o + (unsigned)(j & 1) + (unsigned)((j >> 1) & 1) * st[1] + (unsigned)(j >> 2) * st[2]];
+        }
+        const float inner = primary == 0 ? own[0] : (primary == 1 ? own[1] : own[2]);
+        const bool tp = 2 * Ip + 1 < np;
+        g[i] = 0.0f;
+        fx[i] = s[0];
+        fy[i] = s[1];
+        fz[i] = s[2];
+        t[i] = mg_series(end[0], inner, tp, 0.0f, false) + mg_series(end[1], inner, tp, 0.0f, false);
     }
 }
 
@@ -658,6 +791,55 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_diag(RbLaunch L, MgLaunch M) 
     }
 }
 
+// Inverse of the last level's matrix (-A, at most 64 cells), by Gauss-Jordan elimination without
+// pivoting (the matrix is symmetric and positive definite), stored 64 x 64 with zeros around.
+// Cells cut off from both ends (a phase without conductivity) leave a pivot of rounding size: that
+// row and column are left at zero, which keeps the product symmetric and positive semi-definite.
+constexpr int kMgInv = 64;
+__global__ __launch_bounds__(kMgBottomThreads) void k_mg_inv(MgLaunch M) {
+    __shared__ double a[kMgInv][kMgInv + 1], least[kMgInv];
+    const MgDesc& d = M.vol[M.vols[blockIdx.x]];
+    const MgLevel q = d.lev[d.nlev - 1];
+    const float* t = d.mem + q.off + q.n;
+    const float *fx = t + q.n, *fy = fx + q.n, *fz = fy + q.n;
+    const int tid = (int)threadIdx.x;
+    for (int k = tid; k < kMgInv * kMgInv; k += kMgBottomThreads) a[k / kMgInv][k % kMgInv] = 0.0;
+    __syncthreads();
+    if (tid < q.n) {
+        const int x = tid % q.nx, y = (tid / q.nx) % q.ny, z = tid / (q.nx * q.ny);
+        double diag = t[tid];
+        auto face = [&](bool has, int j, float f) {
+            if (!has) return;
+            a[tid][j] = -(double)f;
+            diag += f;
+        };
+        face(x + 1 < q.nx, tid + 1, fx[tid]);
+        face(x > 0, tid - 1, fx[x > 0 ? tid - 1 : tid]);
+        face(y + 1 < q.ny, tid + q.nx, fy[tid]);
+        face(y > 0, tid - q.nx, fy[y > 0 ? tid - q.nx : tid]);
+        face(z + 1 < q.nz, tid + q.nx * q.ny, fz[tid]);
+        face(z > 0, tid - q.nx * q.ny, fz[z > 0 ? tid - q.nx * q.ny : tid]);
+        a[tid][tid] = diag;
+        least[tid] = 1e-12 * diag;
+    }
+    __syncthreads();
+    const int r = tid >> 4, c0 = 4 * (tid & 15);   // this thread's four elements
+    for (int k = 0; k < q.n; ++k) {
+        const double p = a[k][k] > least[k] ? 1.0 / a[k][k] : 0.0, f = a[r][k];
+        double row[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) row[m] = c0 + m == k ? p : a[k][c0 + m] * p;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 4; ++m) a[r][c0 + m] = r == k ? row[m] : (c0 + m == k ? 0.0 : a[r][c0 + m]) - f * row[m];
+        __syncthreads();
+    }
+    float* out = d.mem + d.inv_off;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        out[r * kMgInv + c0 + m] = r < q.n && c0 + m < q.n ? (float)a[r][c0 + m] : 0.0f;
+}
+
 }  // namespace
 
 bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats) {
@@ -667,7 +849,7 @@ bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats) {
     if ((long long)nx * ny * nz < kMgMinVoxels || flow < kMgMinFlow) return false;
     int x = nx, y = ny, z = nz;
     size_t off = 0;
-    while ((d->nlev == 0 || x > 1 || y > 1 || z > 1) && d->nlev < kMgLevels) {
+    while ((d->nlev == 0 || d->lev[d->nlev - 1].n > kMgInv) && d->nlev < kMgLevels) {
         x = half_up(x);
         y = half_up(y);
         z = half_up(z);
@@ -679,7 +861,10 @@ bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats) {
         l.off = (unsigned)off;
         off += (size_t)kMgArrays * l.n;
     }
-    if (d->lev[d->nlev - 1].n != 1) return false;
+    if (d->lev[d->nlev - 1].n > kMgInv) return false;
+    off = (off + 3) & ~(size_t)3;   // float4 rows
+    d->inv_off = (unsigned)off;
+    off += kMgInv * kMgInv;
     int cells = 0;
     d->bottom = d->nlev;
     while (d->bottom > 0 && cells + d->lev[d->bottom - 1].n <= kMgBottomCells) cells += d->lev[--d->bottom].n;
@@ -699,25 +884,30 @@ bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats) {
 
 hipError_t mg_setup(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {
     if (M.nvol <= 0) return hipSuccess;
-    for (int l = 0; l < M.nlev_max; ++l)
-        hipLaunchKernelGGL(k_mg_coef, dim3(l == 0 ? 512 : (l == 1 ? 64 : 8), M.nvol), dim3(kMgThreads), 0, s, L, M, l);
-    hipLaunchKernelGGL(k_mg_diag, dim3(512, M.nvol), dim3(kMgThreads), 0, s, L, M);
+    auto blocks = [](int cells) { return (unsigned)std::min(32768, std::max(1, (cells + kMgThreads - 1) / kMgThreads)); };
+    hipLaunchKernelGGL(k_mg_coef0, dim3(blocks(M.cells[0]), M.nvol), dim3(kMgThreads), 0, s, L, M);
+    for (int l = 1; l < M.nlev_max; ++l)
+        hipLaunchKernelGGL(k_mg_coef, dim3(blocks(M.cells[l]), M.nvol), dim3(kMgThreads), 0, s, L, M, l);
+    hipLaunchKernelGGL(k_mg_diag, dim3(blocks(M.cells[0]), M.nvol), dim3(kMgThreads), 0, s, L, M);
+    hipLaunchKernelGGL(k_mg_inv, dim3(M.nvol), dim3(kMgBottomThreads), 0, s, M);
     return hipGetLastError();
 }
 
 hipError_t mg_cycle(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {
     const dim3 fb(kRbTX * (kMgTY + 3)), cb(kMgThreads);
+    auto args = [&](int l) {
+        return MgLevelArgs{L.st, M.vol, M.blocks + M.blk_off[l], M.nblk[l], l, L.solo ? M.vol0.mem : nullptr,
+                           M.vol0.lev[l], M.vol0.lev[l + 1]};
+    };
     hipLaunchKernelGGL((k_mg_fine<kMgTY, false>), dim3(M.ntiles), fb, 0, s, L, M);
     for (int l = 0; l < M.nlev; ++l) {
-        const int2* blk = M.blocks + M.blk_off[l];
-        hipLaunchKernelGGL((k_mg_level<MG_PRE_BLACK>), dim3(M.nblk[l]), cb, 0, s, L, M.vol, blk, M.nblk[l], l);
-        hipLaunchKernelGGL((k_mg_level<MG_RESTRICT>), dim3(M.nblk[l]), cb, 0, s, L, M.vol, blk, M.nblk[l], l);
+        hipLaunchKernelGGL((k_mg_level<MG_PRE_BLACK>), dim3(M.nblk[l]), cb, 0, s, args(l));
+        hipLaunchKernelGGL((k_mg_level<MG_RESTRICT>), dim3(M.nblk[l]), cb, 0, s, args(l));
     }
     hipLaunchKernelGGL(k_mg_bottom, dim3(M.nvol), dim3(kMgBottomThreads), 0, s, L, M);
     for (int l = M.nlev - 1; l >= 0; --l) {
-        const int2* blk = M.blocks + M.blk_off[l];
-        hipLaunchKernelGGL((k_mg_level<MG_POST_BLACK>), dim3(M.nblk[l]), cb, 0, s, L, M.vol, blk, M.nblk[l], l);
-        hipLaunchKernelGGL((k_mg_level<MG_POST_RED>), dim3(M.nblk[l]), cb, 0, s, L, M.vol, blk, M.nblk[l], l);
+        hipLaunchKernelGGL((k_mg_level<MG_POST_BLACK>), dim3(M.nblk[l]), cb, 0, s, args(l));
+        hipLaunchKernelGGL((k_mg_level<MG_POST_RED>), dim3(M.nblk[l]), cb, 0, s, args(l));
     }
     hipLaunchKernelGGL((k_mg_fine<kMgTY, true>), dim3(M.ntiles), fb, 0, s, L, M);
     hipLaunchKernelGGL(k_mg_fin, dim3(M.nvol), dim3(kFinThreads), 0, s, L, M);

@@ -972,10 +972,12 @@ void mg_lists(const std::vector<MgDesc>& desc, const std::vector<int>& vols, MgL
     M->nvol = (int)vols.size();
     M->nlev = 0;
     M->nlev_max = 0;
+    for (int& c : M->cells) c = 0;
     for (int v : vols) {
         for (int t = 0; t < desc[v].ntiles; ++t) out->tiles.push_back(int2{v, t});
         M->nlev = std::max(M->nlev, desc[v].bottom);
         M->nlev_max = std::max(M->nlev_max, desc[v].nlev);
+        for (int l = 0; l < desc[v].nlev; ++l) M->cells[l] = std::max(M->cells[l], desc[v].lev[l].n);
     }
     M->ntiles = (int)out->tiles.size();
     for (int l = 0; l < M->nlev; ++l) {
@@ -1199,6 +1201,9 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         B.hrb[i].code_c[0] = codes + B.hrb[i].off_c;
         B.hrb[i].code_c[1] = codes + total_c + B.hrb[i].off_c;
     }
+    L.solo = nv == 1 ? 1 : 0;
+    L.vol0 = B.hrb[0];
+    L.coef0 = B.hcoef[0];
     e = hipMemcpyAsync(m + o_rb, B.hrb.data(), sizeof(RbDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = ft::rb_setup(L, ctx->stream);
     MgLists lists;
@@ -1209,6 +1214,7 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         if (L.staged != 2) B.mg_mem = dalloc(ctx, mg_floats * sizeof(float));
         float* mem = L.staged == 2 ? (float*)L.y : (float*)B.mg_mem;
         for (int i : B.mg_vols) B.hmg[i].mem = L.staged == 2 ? mem + 2 * B.hrb[i].off_c : mem + mg_off[i];
+        M.vol0 = B.hmg[0];
         mg_lists(B.hmg, B.mg_vols, &lists, &M);
         const size_t b_vols = align_up(sizeof(int) * lists.vols.size(), 256);
         const size_t b_tiles = align_up(sizeof(int2) * lists.tiles.size(), 256);

@@ -199,6 +199,11 @@ struct RbDesc {
 
 struct RbLaunch {
     int ntiles, nvol;
+    int solo;         // 1: a launch over one volume, whose descriptor and coefficients are vol0 and coef0 (a
+                      // kernel's first vector loads then wait for one dependent load, not three) and
+                      // whose tiles are the launch's
+    RbDesc vol0;
+    Coef<double> coef0;
     int ty;           // rows per tile (2, 4, 8, 9, 10, 12 or 13) of every red-black pass of this launch set
     int ahead;        // fused Y+Q pass: planes its loads run ahead (2 or 3)
     int staged;       // 2: Y and Q fused (no Y vector); 1: Q pass with the Y planes staged in LDS; 0: six
@@ -243,7 +248,7 @@ inline int rb_row_pitch(int hx) { return (hx + 2 + 3) & ~3; }
 // FP32; the CG around it keeps its FP64 arithmetic, FP64 residuals and stopping rule.
 // A volume whose residual has not dropped to its next reliable update within kMgStall iterations
 // (seen at solid conductivities of 1e-6 and 95% solid) goes on with the Jacobi form from its x64.
-// Level l >= 1 holds, per cell, the right-hand side (overwritten by the solution), the black
+// The last level has at most 64 cells and is solved with its inverse.  Level l >= 1 holds, per cell, the right-hand side (overwritten by the solution), the black
 // values of the first sweep, the face coefficients towards x+, y+ and z+, and 1 / diagonal, all
 // for -A (positive).  Levels from `bottom` on are solved by one block per volume in LDS.
 constexpr int kMgStall = 128;           // iterations without a reliable update before the Jacobi form takes over
@@ -260,10 +265,17 @@ struct MgDesc {
     int nlev, bottom;                   // coarse levels (lev[0] is the fine grid's first coarsening)
     int tiles_x, tiles_y, tiles_z, tz;  // fine tiles of 64 slots x kMgTY rows x tz planes (tz even)
     int ntiles, part_base;
+    unsigned inv_off;                   // floats from mem to the last level's inverse
     float* mem;
     MgLevel lev[kMgLevels];
 };
+struct MgFine {                         // what the fine-level kernels read of a MgDesc
+    int tiles_x, tiles_y, tz, part_base;
+    int cnx, cny;
+    float* g1;
+};
 struct MgLaunch {
+    MgDesc vol0;                        // solo launches (RbLaunch::solo): the volume's descriptor
     int nvol, ntiles;                   // preconditioned volumes, fine tiles
     int nlev, nlev_max;                 // levels launched block-wise; most levels of a volume
     const MgDesc* vol;                  // by volume of the batch
@@ -271,6 +283,7 @@ struct MgLaunch {
     const int2* tiles;                  // fine tiles: (volume, tile of the volume)
     const int2* blocks;                 // coarse-level blocks: (volume, block of its level), level after level
     int blk_off[kMgLevels], nblk[kMgLevels];
+    int cells[kMgLevels];               // most cells of a volume, by level
     double* part;                       // 2 doubles per fine tile: r.z as (hi, lo)
     float* tab;                         // per volume kTabEntries: -1 / diagonal
 };
