@@ -232,7 +232,10 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     fast_ctx* ctx = s->ctx;
     int tiles = 0;
     std::vector<int> tv, mv;
-    int mg_tiles = 0;
+    std::vector<std::array<int, 3>> grids;
+    for (const Req* r : s->slots)
+        if (r) grids.push_back({(r->nx + 1) / 2, r->ny, r->nz});
+    const int btz = rb_batch_tz(ctx, s->rbs.ty, grids);
     for (int i = 0; i < s->max_active; ++i) {
         RbDesc& d = s->h_rb[i];
         Req* r = s->slots[i];
@@ -241,9 +244,7 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
         if (!r) continue;
         size_t floats = 0;
         if (mg_plan(r->nx, r->ny, r->nz, r->prm.dir / 2, &s->h_mg[i], &floats)) {
-            s->h_mg[i].part_base = mg_tiles;
             s->h_mg[i].mem = s->mg_base + 2 * r->off;
-            mg_tiles += s->h_mg[i].ntiles;
             mv.push_back(i);
         }
         d.nx = r->nx;
@@ -257,7 +258,7 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
         d.sgn = (r->prm.dir % 2 == 0) ? 1 : -1;
         d.tiles_x = (d.hx + kRbTX - 1) / kRbTX;
         d.tiles_y = (r->ny + s->rbs.ty - 1) / s->rbs.ty;
-        d.tz = r->tz;
+        d.tz = btz ? btz : r->tz;
         d.tiles_z = (r->nz + d.tz - 1) / d.tz;
         d.ntiles = d.tiles_x * d.tiles_y * d.tiles_z;
         d.off_c = (long long)r->off;
@@ -275,6 +276,7 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     if (!s->d_part || !s->d_partb) return FAST_E_OOM;
     MgLists lists;
     MgLaunch& M = s->ML;
+    const int mg_tiles = mg_tile(s->h_mg, mv);
     mg_lists(s->h_mg, mv, &lists, &M);
     std::vector<int> fresh;   // newly admitted: their levels are built below
     for (Req* r : adm)

@@ -284,6 +284,28 @@ RbShape rb_shape(const fast_ctx* ctx, int nx, int ny, int nz) {
     return r;
 }
 
+int rb_batch_tz(const fast_ctx* ctx, int ty, const std::vector<std::array<int, 3>>& vols) {
+    if (vols.size() < 2) return 0;
+    if (ctx->rb_forced.tz > 0 || std::getenv("FAST_TAU_RB_TZ")) return 0;
+    const long long round = 256ll * std::max(1, 24 / (ty + 3));
+    int best = 0;
+    long long least = 0;
+    for (int tz = 4; tz <= 64; tz += 2) {
+        long long n = 0;
+        int most = 0;
+        for (const auto& v : vols) {
+            n += (long long)((v[0] + kRbTX - 1) / kRbTX) * ((v[1] + ty - 1) / ty) * ((v[2] + tz - 1) / tz);
+            most = std::max(most, std::min(tz, v[2]));
+        }
+        const long long cost = ((n + round - 1) / round) * (most + 3);
+        if (!best || cost < least) {
+            best = tz;
+            least = cost;
+        }
+    }
+    return best;
+}
+
 }  // namespace fth
 
 using namespace fth;
@@ -1013,7 +1035,6 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
     B.hmg.assign(nv, MgDesc{});
     std::vector<size_t> mg_off(nv, 0);
     size_t mg_floats = 0;
-    int mg_tiles = 0;
     B.hrb.resize(nv);
     B.hvol.resize(nv);
     B.hcoef.resize(nv);
@@ -1024,6 +1045,9 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
     for (const Job* j : B.jobs)
         if ((size_t)j->vol->nx * j->vol->ny * j->vol->nz > (size_t)big->nx * big->ny * big->nz) big = j->vol;
     const RbShape bs = rb_shape(ctx, big->nx, big->ny, big->nz);
+    std::vector<std::array<int, 3>> grids;
+    for (const Job* j : B.jobs) grids.push_back({(j->vol->nx + 1) / 2, j->vol->ny, j->vol->nz});
+    const int btz = rb_batch_tz(ctx, bs.ty, grids);
     int tiles = 0, planes = 0;
     size_t total = 0, total_c = 0;
     for (int i = 0; i < nv; ++i) {
@@ -1046,7 +1070,7 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         r.sgn = (j.prm.dir % 2 == 0) ? 1 : -1;
         r.tiles_x = (r.hx + kRbTX - 1) / kRbTX;
         r.tiles_y = (v->ny + bs.ty - 1) / bs.ty;
-        r.tz = rb_shape(ctx, v->nx, v->ny, v->nz).tz;
+        r.tz = btz ? btz : rb_shape(ctx, v->nx, v->ny, v->nz).tz;
         r.tiles_z = (v->nz + r.tz - 1) / r.tz;
         r.tile_base = tiles;
         r.ntiles = r.tiles_x * r.tiles_y * r.tiles_z;
@@ -1087,13 +1111,12 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         if (use_mg && mg_plan(v->nx, v->ny, v->nz, r.primary, &B.hmg[i], &floats)) {
             s.mg = 1;
             s.mg_stall = ctx->mg_stall;
-            B.hmg[i].part_base = mg_tiles;
-            mg_tiles += B.hmg[i].ntiles;
             mg_off[i] = mg_floats;
             mg_floats += align_up(floats, 64);
             B.mg_vols.push_back(i);
         }
     }
+    const int mg_tiles = mg_tile(B.hmg, B.mg_vols);
     B.ntiles = tiles;
     B.nplanes = planes;
     B.htile.resize(tiles);

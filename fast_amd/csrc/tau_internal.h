@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <vector>
 #include <cstddef>
 
 namespace ft {
@@ -264,7 +265,7 @@ struct MgLevel {
 struct MgDesc {
     int nlev, bottom;                   // coarse levels (lev[0] is the fine grid's first coarsening)
     int tiles_x, tiles_y, tiles_z, tz;  // fine tiles of 64 slots x kMgTY rows x tz planes (tz even)
-    int ntiles, part_base;
+    int nz, ntiles, part_base;
     unsigned inv_off;                   // floats from mem to the last level's inverse
     float* mem;
     MgLevel lev[kMgLevels];
@@ -291,6 +292,8 @@ struct MgLaunch {
 // the Jacobi form (the rule depends on the extents alone).  Fills everything but part_base and mem; *floats: level
 // storage, at most 2 floats per element of the padded per-colour layout.
 bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats);
+// Splits the fine grids of the listed volumes, which run together, into tiles; returns their number.
+int mg_tile(std::vector<MgDesc>& d, const std::vector<int>& vols);
 // Level coefficients and FP32 tables (codes and Coef uploaded before).
 hipError_t mg_setup(const RbLaunch&, const MgLaunch&, hipStream_t);
 // z = B r into the buffer of the next p, then beta, for the running volumes that are preconditioned.
