@@ -41,8 +41,9 @@ __device__ __forceinline__ float mg_sum(const FacePair<float>* ftab, int code, c
     return acc;
 }
 
-__device__ __forceinline__ MgFine mg_fine(const MgDesc& d) {
-    return MgFine{d.tiles_x, d.tiles_y, d.tz, d.part_base, d.lev[0].nx, d.lev[0].ny, d.mem + d.lev[0].off};
+// g1: the first level's g (pre), its solution (post).
+__device__ __forceinline__ MgFine mg_fine(const MgDesc& d, bool post) {
+    return MgFine{d.tiles_x, d.tiles_y, d.tz, d.part_base, d.lev[0].nx, d.lev[0].ny, d.mem + d.lev[0].off + (post ? d.lev[0].n : 0)};
 }
 
 // Fine level.  Geometry, rings and LDS planes as in k_rb_yq (columns that march z, p planes
@@ -72,9 +73,9 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
     const RbDesc d = rb_desc(L, v);
     MgFine md;
     if (L.solo)
-        md = mg_fine(M.vol0);
+        md = mg_fine(M.vol0, POST);
     else
-        md = mg_fine(M.vol[v]);
+        md = mg_fine(M.vol[v], POST);
     md = uniform(md);
     __shared__ float tab[kTabEntries];
     __shared__ FacePair<float> ftab[8];
@@ -266,51 +267,11 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
 }
 
 // ---- coarse levels -------------------------------------------------------------------------
-// A thread takes the red or black voxel of one row of one coarse cell: four consecutive lanes
-// (the cell's four rows) per cell of the next level, so the restriction sums four lanes.
-struct MgLev {
-    int nx, ny, nz, cx, cy;          // extents; those of the next level (x, y)
-    float *g, *t, *fx, *fy, *fz, *iv;
-    float* gc;                       // next level's g
-};
-
-__device__ __forceinline__ MgLev mg_lev(const MgLevel& a, const MgLevel& c, float* mem) {
-    MgLev r;
-    r.nx = a.nx;
-    r.ny = a.ny;
-    r.nz = a.nz;
-    r.cx = half_up(a.nx);
-    r.cy = half_up(a.ny);
-    r.g = mem + a.off;
-    r.t = r.g + a.n;
-    r.fx = r.t + a.n;
-    r.fy = r.fx + a.n;
-    r.fz = r.fy + a.n;
-    r.iv = r.fz + a.n;
-    r.gc = mem + c.off;
-    return r;
-}
-
 struct MgCell {
     int x, y, z;
     unsigned i;
     bool ok;
 };
-
-// Cell of colour `colour` in row j (0..3) of coarse cell C.
-__device__ __forceinline__ MgCell mg_cell(int nx, int ny, int nz, int cx, int cy, unsigned C, int j, int colour) {
-    const unsigned row = C / (unsigned)cx;
-    const int K = (int)(C - row * (unsigned)cx);
-    const int Z = (int)(row / (unsigned)cy), Y = (int)(row - (unsigned)Z * (unsigned)cy);
-    MgCell c;
-    c.y = 2 * Y + (j & 1);
-    c.z = 2 * Z + (j >> 1);
-    c.x = 2 * K + ((colour + c.y + c.z) & 1);
-    c.ok = c.x < nx && c.y < ny && c.z < nz;
-    if (!c.ok) c.x = c.y = c.z = 0;   // a cell in the box: its neighbours' indices stay inside too
-    c.i = (unsigned)c.x + (unsigned)nx * ((unsigned)c.y + (unsigned)ny * (unsigned)c.z);
-    return c;
-}
 
 // Face coefficients and indices of the six neighbours (x-, x+, y-, y+, z-, z+); a face of the box
 // has coefficient 0 and the cell itself as neighbour.
@@ -344,20 +305,41 @@ struct MgLevelArgs {
     const VolState<double>* st;
     const MgDesc* vol;
     const int2* blocks;
-    int nblk, lev;
+    int nblk, lev, tz;
     float* mem;         // solo launches: the volume's level storage, this level and the next
     MgLevel la, lc;
 };
 
-enum MgStep : int { MG_PRE_BLACK = 0, MG_RESTRICT, MG_POST_BLACK, MG_POST_RED };
+struct Float2 {   // two neighbouring floats at any element
+    float x, y;
+};
+__device__ __forceinline__ Float2 ld2(const float* p, unsigned i) {
+    Float2 v;
+    __builtin_memcpy(&v, p + i, sizeof(v));
+    return v;
+}
 
-// Half sweeps of one level:
-//   pre black:  t = (g + sum c g_r iv_r) iv on black cells (red ones: g iv, never stored)
-//   restrict:   next g = sum over the cell's red children of sum c t_b
-//   post black: g = (g + sum c (g_r iv_r + e)) iv on black cells, e the next level's solution
-//   post red:   g = (g + sum c g_b) iv on red cells (g is then the level's solution)
-template <int STEP>
+// One level, half a cycle per launch:
+//   down: b = (g + sum c g_r iv_r) iv on the black cells (the red ones are g iv), next g = sum over the
+//         cell's red children of sum c b
+//   up:   b = (g + sum c (g_r iv_r + e)) iv with e the next level's solution (its t), red cells
+//         (g + sum c b) iv; both are the level's solution, stored in t
+// A thread takes a column of cell pairs (2k, 2k + 1) of one row and marches z; each plane of a pair has
+// one red and one black cell.  Step t forms the black cells of plane t and the red ones of plane t - 1,
+// which are at the same x.  LDS holds a value per pair: the red values of planes t, t + 1 and the black
+// ones of planes t - 1, t.  A tile has one pair and two rows of halo on each side, where the values
+// its own red cells need are formed again.  Loads take both cells of a pair, two planes ahead.
+// Bound by the chain of steps at 32^3 and 64^3 cells, by loads and memory (five values a cell) beyond.
+// Two launches a half cycle, one per colour with a thread per cell of that colour, took twice the
+// traffic: a cycle's levels of 64^3 (one level) 15.4 -> 9.8 us in half as many launches, of 256^3
+// (three) 75 -> 61 us, of 384^3 (four) 197 -> 151 us, of 24 volumes 100 -> 88 us.  With 4-byte loads
+// of the cells' own faces this form took 83 us at 256^3; tiles of 24 rows and 512 threads are even.
+template <bool UP>
 __global__ __launch_bounds__(kMgThreads) void k_mg_level(MgLevelArgs A) {
+    constexpr int TK = kMgLevTK, TY = kMgLevTY, PW = TK + 2, PH = TY + 4;
+    static_assert(PW * PH <= kMgThreads && TY % 2 == 0, "a thread per pair of the tile and its halo");
+    __shared__ float wbuf[2][PW * (PH + 2) + 2], bbuf[2][PW * (PH + 2) + 2];
+    __shared__ float rows[2][TY / 2][TK];
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= A.nblk) return;
     int2 b{0, slot};
@@ -371,58 +353,130 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_level(MgLevelArgs A) {
     }
     if (A.st[b.x].status != ST_RUNNING || !A.st[b.x].mg) return;
     b = uniform(b);
-    const MgLev l = mg_lev(uniform(la), uniform(lc), uniform(mem));
-    const unsigned id = (unsigned)b.y * kMgThreads + threadIdx.x;
-    const unsigned C = id >> 2, nc = (unsigned)lc.n;
-    constexpr int colour = (STEP == MG_PRE_BLACK || STEP == MG_POST_BLACK) ? 1 : 0;
-    MgCell c = mg_cell(l.nx, l.ny, l.nz, l.cx, l.cy, C < nc ? C : 0u, (int)(id & 3u), colour);
-    c.ok = c.ok && C < nc;
-    float f[6];
-    unsigned n[6];
-    mg_faces(l, c, f, n);
-    float u[6];
-    if (STEP == MG_RESTRICT) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k) u[k] = l.t[n[k]];
-        float s = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) u[k] = f[k] != 0.0f ? u[k] : 0.0f;   // a box face's "neighbour" is red
-        s = c.ok ? mg_dot(f, u) : 0.0f;
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
-        if ((id & 3u) == 0u && C < nc) l.gc[C] = s;
-        return;
-    }
-#pragma unroll
-    for (int k = 0; k < 6; ++k) u[k] = l.g[n[k]];
-    if (STEP != MG_POST_RED) {
-        float w[6];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) w[k] = l.iv[n[k]];
-        if (STEP == MG_POST_BLACK) {
-            float e[6];
-            const unsigned px = (unsigned)l.cx, pxy = (unsigned)l.cx * (unsigned)l.cy;
-            const unsigned cb = (unsigned)(c.y >> 1) * px + (unsigned)(c.z >> 1) * pxy;
-            const unsigned base = cb + (unsigned)(c.x >> 1);
-            e[0] = l.gc[c.x > 0 ? cb + (unsigned)((c.x - 1) >> 1) : base];
-            e[1] = l.gc[c.x + 1 < l.nx ? cb + (unsigned)((c.x + 1) >> 1) : base];
-            e[2] = l.gc[c.y > 0 && !(c.y & 1) ? base - px : base];
-            e[3] = l.gc[c.y + 1 < l.ny && (c.y & 1) ? base + px : base];
-            e[4] = l.gc[c.z > 0 && !(c.z & 1) ? base - pxy : base];
-            e[5] = l.gc[c.z + 1 < l.nz && (c.z & 1) ? base + pxy : base];
-#pragma unroll
-            for (int k = 0; k < 6; ++k) u[k] = fmaf(u[k], w[k], e[k]);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 6; ++k) u[k] = u[k] * w[k];
+    la = uniform(la);
+    lc = uniform(lc);
+    mem = uniform(mem);
+    const int nx = la.nx, ny = la.ny, nz = la.nz, cx = lc.nx, cy = lc.ny;
+    const unsigned nxy = (unsigned)nx * (unsigned)ny, cxy = (unsigned)cx * (unsigned)cy;
+    const float* G = mem + la.off;
+    float* S = mem + la.off + la.n;   // t
+    const float *FX = S + la.n, *FY = FX + la.n, *FZ = FY + la.n, *IV = FZ + la.n;
+    float* GC = mem + lc.off;         // next level: g (down), t (up)
+    const float* E = GC + lc.n;
+    const int tx = (cx + TK - 1) / TK, ty = (ny + TY - 1) / TY;
+    const int k0 = (b.y % tx) * TK, y0 = ((b.y / tx) % ty) * TY, z0 = (b.y / (tx * ty)) * A.tz;
+    const int z1 = min(z0 + A.tz, nz);
+    const int tid = (int)threadIdx.x;
+    const bool has = tid < PW * PH;
+    const int ck = tid % PW, cr = tid / PW;
+    const int k = k0 - 1 + ck, y = y0 - 2 + cr;
+    const bool inb = has && k >= 0 && k < cx && y >= 0 && y < ny;
+    const bool ok0 = inb && 2 * k < nx, ok1 = inb && 2 * k + 1 < nx;
+    const bool mid = has && cr >= 1 && cr <= TY + 2;                               // black values are formed here
+    const bool own = has && ck >= 1 && ck <= TK && cr >= 2 && cr < TY + 2;
+    // place in LDS, with a row of padding on either side; threads without a pair write the spare place
+    const int at = has ? PW + 1 + tid : PW * (PH + 2) + 1, rd = has ? at : PW + 1;
+    const unsigned col = inb ? 2u * (unsigned)k + (unsigned)nx * (unsigned)y : 0u;
+    const unsigned colx = inb && k > 0 ? col - 1u : 0u, coly = inb && y > 0 ? col - (unsigned)nx : 0u;
+    const unsigned ccol = inb ? (unsigned)k + (unsigned)cx * (unsigned)(y >> 1) : 0u;
+    auto plane = [&](int z) { return (unsigned)min(max(z, 0), nz - 1) * nxy; };
+    // both cells of the pair on one plane (the second one of a row's last pair may be the next value
+    // in memory: it is never used)
+    struct Pair {
+        Float2 g, iv, fx, fy, fz, ym;
+        float xm, e;
+    };
+    Pair ring[4];   // planes t - 1 .. t + 2
+    auto load = [&](Pair& q, int z) {
+        const unsigned o = plane(z);
+        q.g = ld2(G + o, col);
+        q.iv = ld2(IV + o, col);
+        q.fx = ld2(FX + o, col);
+        q.fy = ld2(FY + o, col);
+        q.fz = ld2(FZ + o, col);
+        q.ym = ld2(FY + o, coly);
+        q.xm = FX[o + colx];
+        if (UP) q.e = E[(unsigned)(min(max(z, 0), nz - 1) >> 1) * cxy + ccol];
+    };
+    // by masks: a choice between two fields becomes an access with a computed address, in scratch memory
+    auto pick = [](Float2 v, int s) {
+        const unsigned m = 0u - (unsigned)s;
+        return __uint_as_float((__float_as_uint(v.x) & ~m) | (__float_as_uint(v.y) & m));
+    };
+    auto ok = [&](int s) { return s ? ok1 : ok0; };
+    // value of the red cell of plane z, at parity s
+    auto red_value = [&](const Pair& q, int z, int s) {
+        const float g = pick(q.g, s), iv = pick(q.iv, s);
+        const float v = UP ? fmaf(g, iv, q.e) : g * iv;
+        return ok(s) && (unsigned)z < (unsigned)nz ? v : 0.0f;
+    };
+    // sum of face times neighbour of the cell at parity s of plane z; zm: faces of plane z - 1
+    auto dot = [&](const Pair& q, const Float2& zm, int z, int s, const float (&u)[6]) {
+        const float xm = k > 0 ? q.xm : 0.0f;
+        const float f[6] = {pick(Float2{xm, q.fx.x}, s), pick(q.fx, s), y > 0 ? pick(q.ym, s) : 0.0f, pick(q.fy, s),
+                            z > 0 ? pick(zm, s) : 0.0f, pick(q.fz, s)};
+        return mg_dot(f, u);
+    };
+    const int t0 = z0 - 1;
+    load(ring[3], t0 - 1);
+    load(ring[0], t0);
+    load(ring[1], t0 + 1);
+    const int sy = (1 + y) & 1;   // parity of the row's black cells in even planes
+    float wm = red_value(ring[3], t0 - 1, sy ^ (t0 & 1)), w0 = red_value(ring[0], t0, 1 ^ sy ^ (t0 & 1));
+    float bm = 0.0f, b1 = 0.0f;   // black values of planes t - 2 and t - 1 in this column
+    float hold = 0.0f;            // down: the pair of planes' first sum
+    auto step = [&](auto J, int t) {
+        constexpr int j = decltype(J)::value, jm = (j + 3) % 4, jp = (j + 1) % 4, jn = (j + 2) % 4;
+        const int s = sy ^ (t & 1);
+        const Float2 zz = ring[jn].fz;   // plane t - 2
+        load(ring[jn], t + 2);
+        const float wp = red_value(ring[jp], t + 1, s);
+        wbuf[t & 1][at] = w0;
+        __syncthreads();
+        const float* w = wbuf[t & 1] + rd;
+        float bv;
+        {
+            const float u[6] = {w[s - 1], w[s], w[-PW], w[PW], wm, wp};
+            bv = (pick(ring[j].g, s) + dot(ring[j], ring[jm].fz, t, s, u)) * pick(ring[j].iv, s);
+            bv = mid && ok(s) && (unsigned)t < (unsigned)nz ? bv : 0.0f;
         }
-    }
-    const float r = (l.g[c.i] + mg_dot(f, u)) * l.iv[c.i];
-    if (!c.ok) return;
-    if (STEP == MG_PRE_BLACK)
-        l.t[c.i] = r;
-    else
-        l.g[c.i] = r;
+        bbuf[t & 1][at] = bv;
+        const int tq = t - 1;
+        float d = 0.0f;
+        if (own && ok(s) && tq >= z0) {
+            const float* bl = bbuf[(t & 1) ^ 1] + rd;
+            const float u[6] = {bl[s - 1], bl[s], bl[-PW], bl[PW], bm, bv};
+            d = dot(ring[jm], zz, tq, s, u);
+        }
+        if (UP) {
+            if (own && ok(s)) {
+                if (t >= z0 && t < z1) S[plane(t) + col + (unsigned)s] = bv;
+                if (tq >= z0) S[plane(tq) + col + (unsigned)s] = (pick(ring[jm].g, s) + d) * pick(ring[jm].iv, s);
+            }
+        } else if (tq >= z0) {
+            const int o = tq - z0;
+            if (o & 1) {   // the pair of planes is complete: odd rows hand theirs over
+                hold += d;
+                if (own && (cr & 1)) rows[(o >> 1) & 1][(cr - 2) >> 1][ck - 1] = hold;
+            } else {
+                if (o >= 2 && own && !(cr & 1) && inb)   // after the barrier: the previous pair
+                    GC[(unsigned)((tq - 2) >> 1) * cxy + ccol] = hold + rows[((o >> 1) - 1) & 1][(cr - 2) >> 1][ck - 1];
+                hold = d;
+            }
+        }
+        wm = w0;
+        w0 = wp;
+        bm = b1;
+        b1 = bv;
+    };
+    for (int t = t0;; t += 4)
+        if (ring_turn<0, 4, 4>(step, t, z1)) break;
+    if (UP) return;
+    const int ol = z1 - 1 - z0;   // the last pair (one plane at the end of an odd level)
+    if (own && (cr & 1) && !(ol & 1)) rows[(ol >> 1) & 1][(cr - 2) >> 1][ck - 1] = hold;
+    __syncthreads();
+    if (own && !(cr & 1) && inb)
+        GC[(unsigned)((z1 - 1) >> 1) * cxy + ccol] = hold + rows[(ol >> 1) & 1][(cr - 2) >> 1][ck - 1];
 }
 
 // The levels from `bottom` on, one block per volume, in LDS: one V-cycle with two sweeps before
@@ -595,7 +649,7 @@ __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLa
         sweep(q, 0);
     }
     const float* u = sm[1];
-    for (int i = tid; i < sl[b].n; i += kMgBottomThreads) mem[off_b + i] = u[i];
+    for (int i = tid; i < sl[b].n; i += kMgBottomThreads) mem[off_b + (unsigned)sl[b].n + i] = u[i];
 }
 
 // r.z of one preconditioned volume, then beta = r.z / (previous r.z).
@@ -847,6 +901,8 @@ __global__ __launch_bounds__(kMgBottomThreads) void k_mg_inv(MgLaunch M) {
 // blocks per CU for each volume alone, at most 32 planes: 12 volumes of 60^3 to 129^3 11.8 -> 10.4 ms,
 // 384^3 30.2 -> 29.7 ms.  The choice is within 2% of the best of a sweep over 2 .. 128 for 64^3 to 384^3.
 constexpr int kMgRound = 512;
+// The same for a level's tiles of four waves (four blocks on a CU).
+constexpr int kMgLevRound = 1024;
 
 bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats) {
     *d = MgDesc{};
@@ -883,23 +939,53 @@ bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats) {
     return true;
 }
 
-int mg_tile(std::vector<MgDesc>& d, const std::vector<int>& vols) {
-    auto count = [&](const MgDesc& m, int tz) { return (long long)m.tiles_x * m.tiles_y * ((m.nz + tz - 1) / tz); };
-    int best = 4;
+// The planes per tile with the fewest steps over rounds of `round` blocks; count(tz), most(tz): tiles and
+// planes of the deepest one.
+template <class C, class D>
+static int least_steps(int round, C count, D most) {
+    int best = 2;
     long long least = 0;
     for (int tz = 2; tz <= 128; tz += 2) {
-        long long n = 0;
-        int most = 0;
-        for (int v : vols) {
-            n += count(d[v], tz);
-            most = std::max(most, std::min(tz, d[v].nz));
-        }
-        const long long cost = ((n + kMgRound - 1) / kMgRound) * (most + 3);
+        const long long cost = ((count(tz) + round - 1) / round) * (most(tz) + 3);
         if (tz == 2 || cost < least) {
             best = tz;
             least = cost;
         }
     }
+    return best;
+}
+
+int mg_level_tiles(const MgLevel& l, int tz) {
+    return ((half_up(l.nx) + kMgLevTK - 1) / kMgLevTK) * ((l.ny + kMgLevTY - 1) / kMgLevTY) * ((l.nz + tz - 1) / tz);
+}
+
+int mg_level_tz(const std::vector<MgLevel>& l) {
+    auto count = [&](int tz) {
+        long long n = 0;
+        for (const MgLevel& m : l) n += mg_level_tiles(m, tz);
+        return n;
+    };
+    auto most = [&](int tz) {
+        int n = 0;
+        for (const MgLevel& m : l) n = std::max(n, std::min(tz, m.nz));
+        return n;
+    };
+    return least_steps(kMgLevRound, count, most);
+}
+
+int mg_tile(std::vector<MgDesc>& d, const std::vector<int>& vols) {
+    auto count = [&](const MgDesc& m, int tz) { return (long long)m.tiles_x * m.tiles_y * ((m.nz + tz - 1) / tz); };
+    auto all = [&](int tz) {
+        long long n = 0;
+        for (int v : vols) n += count(d[v], tz);
+        return n;
+    };
+    auto most = [&](int tz) {
+        int n = 0;
+        for (int v : vols) n = std::max(n, std::min(tz, d[v].nz));
+        return n;
+    };
+    const int best = least_steps(kMgRound, all, most);
     int tiles = 0;
     for (int v : vols) {
         MgDesc& m = d[v];
@@ -926,19 +1012,13 @@ hipError_t mg_setup(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {
 hipError_t mg_cycle(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {
     const dim3 fb(kRbTX * (kMgTY + 3)), cb(kMgThreads);
     auto args = [&](int l) {
-        return MgLevelArgs{L.st, M.vol, M.blocks + M.blk_off[l], M.nblk[l], l, L.solo ? M.vol0.mem : nullptr,
+        return MgLevelArgs{L.st, M.vol, M.blocks + M.blk_off[l], M.nblk[l], l, M.lev_tz[l], L.solo ? M.vol0.mem : nullptr,
                            M.vol0.lev[l], M.vol0.lev[l + 1]};
     };
     hipLaunchKernelGGL((k_mg_fine<kMgTY, false>), dim3(M.ntiles), fb, 0, s, L, M);
-    for (int l = 0; l < M.nlev; ++l) {
-        hipLaunchKernelGGL((k_mg_level<MG_PRE_BLACK>), dim3(M.nblk[l]), cb, 0, s, args(l));
-        hipLaunchKernelGGL((k_mg_level<MG_RESTRICT>), dim3(M.nblk[l]), cb, 0, s, args(l));
-    }
+    for (int l = 0; l < M.nlev; ++l) hipLaunchKernelGGL(k_mg_level<false>, dim3(M.nblk[l]), cb, 0, s, args(l));
     hipLaunchKernelGGL(k_mg_bottom, dim3(M.nvol), dim3(kMgBottomThreads), 0, s, L, M);
-    for (int l = M.nlev - 1; l >= 0; --l) {
-        hipLaunchKernelGGL((k_mg_level<MG_POST_BLACK>), dim3(M.nblk[l]), cb, 0, s, args(l));
-        hipLaunchKernelGGL((k_mg_level<MG_POST_RED>), dim3(M.nblk[l]), cb, 0, s, args(l));
-    }
+    for (int l = M.nlev - 1; l >= 0; --l) hipLaunchKernelGGL(k_mg_level<true>, dim3(M.nblk[l]), cb, 0, s, args(l));
     hipLaunchKernelGGL((k_mg_fine<kMgTY, true>), dim3(M.ntiles), fb, 0, s, L, M);
     hipLaunchKernelGGL(k_mg_fin, dim3(M.nvol), dim3(kFinThreads), 0, s, L, M);
     return hipGetLastError();

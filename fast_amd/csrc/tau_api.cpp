@@ -1004,9 +1004,13 @@ void mg_lists(const std::vector<MgDesc>& desc, const std::vector<int>& vols, MgL
     M->ntiles = (int)out->tiles.size();
     for (int l = 0; l < M->nlev; ++l) {
         M->blk_off[l] = (int)out->blocks.size();
+        std::vector<MgLevel> levels;
+        for (int v : vols)
+            if (l < desc[v].bottom) levels.push_back(desc[v].lev[l]);
+        M->lev_tz[l] = mg_level_tz(levels);
         for (int v : vols) {
             if (l >= desc[v].bottom) continue;
-            const int nb = (int)((4ll * desc[v].lev[l + 1].n + kMgThreads - 1) / kMgThreads);
+            const int nb = mg_level_tiles(desc[v].lev[l], M->lev_tz[l]);
             for (int b = 0; b < nb; ++b) out->blocks.push_back(int2{v, b});
         }
         M->nblk[l] = (int)out->blocks.size() - M->blk_off[l];

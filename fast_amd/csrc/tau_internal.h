@@ -257,7 +257,8 @@ constexpr int kMgLevels = 20;           // levels of the coarsest hierarchy a so
 constexpr int kMgArrays = 6;            // g, t, cx, cy, cz, iv
 constexpr int kMgBottomCells = 5120;    // cells of the levels the one-block kernel keeps in LDS
 constexpr int kMgTY = 8;                // rows per fine tile (even: a tile holds whole coarse cells)
-constexpr int kMgThreads = 256;         // threads of a coarse-level block (4 per coarse cell)
+constexpr int kMgThreads = 256;
+constexpr int kMgLevTK = 16, kMgLevTY = 10;   // a level's tile: pairs of cells in x, rows
 struct MgLevel {
     int nx, ny, nz, n;
     unsigned off;                       // floats from MgDesc::mem to the level's arrays
@@ -282,8 +283,8 @@ struct MgLaunch {
     const MgDesc* vol;                  // by volume of the batch
     const int* vols;                    // the preconditioned volumes
     const int2* tiles;                  // fine tiles: (volume, tile of the volume)
-    const int2* blocks;                 // coarse-level blocks: (volume, block of its level), level after level
-    int blk_off[kMgLevels], nblk[kMgLevels];
+    const int2* blocks;                 // coarse-level tiles: (volume, tile of its level), level after level
+    int blk_off[kMgLevels], nblk[kMgLevels], lev_tz[kMgLevels];   // planes per tile of a level
     int cells[kMgLevels];               // most cells of a volume, by level
     double* part;                       // 2 doubles per fine tile: r.z as (hi, lo)
     float* tab;                         // per volume kTabEntries: -1 / diagonal
@@ -294,6 +295,9 @@ struct MgLaunch {
 bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats);
 // Splits the fine grids of the listed volumes, which run together, into tiles; returns their number.
 int mg_tile(std::vector<MgDesc>& d, const std::vector<int>& vols);
+// The same for one level of several volumes: planes per tile, tiles of a volume.
+int mg_level_tz(const std::vector<MgLevel>& l);
+int mg_level_tiles(const MgLevel& l, int tz);
 // Level coefficients and FP32 tables (codes and Coef uploaded before).
 hipError_t mg_setup(const RbLaunch&, const MgLaunch&, hipStream_t);
 // z = B r into the buffer of the next p, then beta, for the running volumes that are preconditioned.
