@@ -26,8 +26,7 @@ hipError_t mesh_emit(const uint8_t* padded, int nx, int ny, int nz, float iso, c
                      const uint64_t* offset, float* out, hipStream_t s);
 }  // namespace fta
 namespace ftc {
-hipError_t ccl_face_codes(const uint32_t* L, long long n, const uint8_t* table, uint32_t numLabels, uint8_t* out,
-                          hipStream_t s);
+hipError_t ccl_face_codes(const uint32_t* L, long long n, uint8_t* table, uint32_t numLabels, uint8_t* out, hipStream_t s);
 }  // namespace ftc
 
 using namespace fth;
