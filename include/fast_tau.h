@@ -114,7 +114,8 @@ typedef struct fast_ctx fast_ctx;
  * batch of large volumes runs in (0 = always one launch; results are the same either way);
  * FAST_TAU_UPDATE_EVERY (default 4) is the number of mixed-form iterations between launches of
  * the reliable-update step (results are the same for every value); FAST_TAU_RB_TZ forces the
- * z depth of the red-black tiles (default: nz * tiles per plane / 2048, clamped to 4..32);
+ * z depth of the red-black tiles (default: the tuned one, else nz * tiles per plane / 2048, clamped
+ * to 4..32; one for all volumes of a batch, from the rounds of the launch);
  * FAST_TAU_MG_STALL (default 128) is the number of multigrid-preconditioned iterations without a
  * reliable update after which a mixed CG solve goes on with the Jacobi preconditioner;
  * FAST_TAU_RB_STAGED=0 selects the red-black Q pass that reads its Y neighbours from memory
