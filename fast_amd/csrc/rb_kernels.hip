@@ -575,7 +575,7 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
     AccDD acc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i].init();
-    if (ps.row_ok) {
+    if (!kTables && ps.row_ok) {
         for (int z = ps.z0; z < ps.z1; ++z) {
             const int s = (kColour + ps.y + z) & 1;
             const int x = 2 * ps.k + s;
@@ -603,12 +603,41 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
                     X64[ci] = X64[ci] + (double)xv;
                 }
                 X[ci] = 0.0f;
-                continue;
             }
-            const int code = ld(d.code_c[kColour], ci);
-            const int bx = box_flags(x, ps.y, z, d.nx, d.ny, d.nz);
+        }
+    }
+    if (kTables) {
+        const unsigned c00 = rb_index(d, 0, 0, 0);
+        const int y = ps.y, k = ps.k;
+        auto parity = [=](int z) { return (kColour + y + z) & 1; };
+        auto valid = [=](int z) { return ps.row_ok && z < ps.z1 && 2 * k + ((kColour + y + z) & 1) < d.nx; };
+        struct In {
+            int code;
+            double x, o[6];   // x64 of the voxel (R64); its neighbours
+        };
+        auto load = [&](int z, In& in) {
+            const int s = parity(z);
+            const unsigned ci = valid(z) ? rb_index(d, k, y, z) : c00;
+            in.code = ld(d.code_c[kColour], ci);
+            if (KIND == RB_R64) {
+                rb_nbrs(X64B, d, ci, s, in.o);
+                in.x = ld(X64, ci);   // not used on the first update
+            } else {
+                rb_nbrs(X64, d, ci, s, in.o);   // not used on the first update
+            }
+        };
+        auto proc = [&](int z, const In& in) {
+            if (!valid(z)) return;
+            const int x = 2 * k + parity(z);
+            const unsigned ci = rb_index(d, k, y, z);
+            const int code = in.code;
+            const int bx = box_flags(x, y, z, d.nx, d.ny, d.nz);
             const DiagInv<double> di = diag_at<double>(tabs.tab, code, bx, d.primary, c);
-            const int kp = d.primary == 0 ? x : (d.primary == 1 ? ps.y : z);
+            const int kp = d.primary == 0 ? x : (d.primary == 1 ? y : z);
+            // rhs_of, its end value by masks: a choice between the fields becomes an access to scratch memory
+            const double b = kp == 0 || kp == nprim - 1
+                                 ? 0.0 - pick2(((code >> 6) & 1) != 0, c.cb0, c.cb1) * pick2(kp == 0, c.cend, c.cbeg)
+                                 : 0.0;
             if (KIND == RB_Y64) {
                 double g;
                 if (first_res) {
@@ -618,31 +647,25 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
                     const FacePair<double> pz = tabs.ftab[((code >> 4) & 3) | o4];
                     auto x0n = [&](int dxp, int dyp, int dzp, bool ok) {
                         if (!ok) return 0.0;
-                        const int kk = d.primary == 0 ? x + dxp : (d.primary == 1 ? ps.y + dyp : z + dzp);
+                        const int kk = d.primary == 0 ? x + dxp : (d.primary == 1 ? y + dyp : z + dzp);
                         return x0_of<double>(kk, nprim, d.sgn);
                     };
                     g = 0.0;
                     g += pz.m * x0n(0, 0, -1, z > 0);
-                    g += py.m * x0n(0, -1, 0, ps.y > 0);
+                    g += py.m * x0n(0, -1, 0, y > 0);
                     g += px.m * x0n(-1, 0, 0, x > 0);
                     g += px.p * x0n(1, 0, 0, x + 1 < d.nx);
-                    g += py.p * x0n(0, 1, 0, ps.y + 1 < d.ny);
+                    g += py.p * x0n(0, 1, 0, y + 1 < d.ny);
                     g += pz.p * x0n(0, 0, 1, z + 1 < d.nz);
                 } else {
-                    double o[6];
-                    rb_nbrs(X64, d, ci, s, o);
-                    g = rb_sum(tabs.ftab, code, o);
+                    g = rb_sum(tabs.ftab, code, in.o);
                 }
-                const double b = rhs_of<double>(code, kp, nprim, c);
                 st(X64B, ci, (b - g) / di.d);
                 acc[0].add(b, b);
-            } else if (KIND == RB_R64) {
-                const double xr = first_res ? x0_of<double>(kp, nprim, d.sgn) : ld(X64, ci);
+            } else {
+                const double xr = first_res ? x0_of<double>(kp, nprim, d.sgn) : in.x;
                 if (first_res) st(X64, ci, xr);
-                const double b = rhs_of<double>(code, kp, nprim, c);
-                double o[6];
-                rb_nbrs(X64B, d, ci, s, o);
-                const double r64 = (b - di.d * xr) - rb_sum(tabs.ftab, code, o);
+                const double r64 = (b - di.d * xr) - rb_sum(tabs.ftab, code, in.o);
                 const float r32 = (float)r64;
                 st(Rr, ci, r32);
                 if (mg) st(L.q + d.off_c, ci, (float)(di.iv * (double)r32));   // x1 of the next cycle
@@ -650,6 +673,19 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
                 acc[1].add(b, b);
                 acc[2].add(r32, r32);
                 acc[3].add((double)r32, di.iv * (double)r32);
+            }
+        };
+        // loads two planes ahead, as in k_rb_it (one plane at a time, each waiting for its loads: 384^3 Y64
+        // 48 and R64 60 us over the launches of a solve, so 41 and 46)
+        constexpr int AH = 2, R = AH + 1;
+        In in[R];
+#pragma unroll
+        for (int i = 0; i < AH; ++i) load(ps.z0 + i, in[i]);
+        for (int z = ps.z0; z < ps.z1; z += R) {
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                load(z + j + AH, in[(j + AH) % R]);
+                proc(z + j, in[j]);
             }
         }
     }
