@@ -943,11 +943,11 @@ bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats) {
 // planes of the deepest one.
 template <class C, class D>
 static int least_steps(int round, C count, D most) {
-    int best = 2;
+    int best = kMgLeastTz;
     long long least = 0;
-    for (int tz = 2; tz <= 128; tz += 2) {
+    for (int tz = kMgLeastTz; tz <= 128; tz += 2) {
         const long long cost = ((count(tz) + round - 1) / round) * (most(tz) + 3);
-        if (tz == 2 || cost < least) {
+        if (tz == kMgLeastTz || cost < least) {
             best = tz;
             least = cost;
         }

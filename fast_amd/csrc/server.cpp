@@ -311,7 +311,7 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     }
     if (e == hipSuccess && M.nvol) {
         e = hipMemcpyAsync(s->d_mg, s->h_mg.data(), sizeof(MgDesc) * s->max_active, hipMemcpyHostToDevice, st);
-        if (e == hipSuccess) e = mg_upload(M, lists, st);
+        if (e == hipSuccess) e = mg_upload(M, lists, lists.blocks.size(), st);   // as many as the block was grown for
         if (e == hipSuccess && !fresh.empty())
             e = hipMemcpyAsync(const_cast<int*>(M.vols) + mv.size(), fresh.data(), sizeof(int) * fresh.size(),
                                hipMemcpyHostToDevice, st);

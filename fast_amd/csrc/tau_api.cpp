@@ -974,6 +974,7 @@ struct RbBatch {
     std::vector<int> mg_vols;    // preconditioned volumes
     MgLaunch M{};
     void* mg_list = nullptr;     // launch lists on the device
+    size_t mg_room = 0;          // blocks that fit there
     void* mg_mem = nullptr;      // level storage where the Y vector is in use (separate Y and Q passes)
 
     ~RbBatch() {
@@ -1017,8 +1018,17 @@ void mg_lists(const std::vector<MgDesc>& desc, const std::vector<int>& vols, MgL
     }
 }
 
-// The launch lists to the device (where M points).
-hipError_t mg_upload(const MgLaunch& M, const MgLists& l, hipStream_t s) {
+size_t mg_list_room(const std::vector<MgDesc>& desc, const std::vector<int>& vols) {
+    size_t n = 0;
+    for (int v : vols)
+        for (int l = 0; l < desc[v].bottom; ++l) n += (size_t)mg_level_tiles(desc[v].lev[l], kMgLeastTz);
+    return n;
+}
+
+hipError_t mg_upload(const MgLaunch& M, const MgLists& l, size_t room, hipStream_t s) {
+    if ((const char*)(M.vols + l.vols.size()) > (const char*)M.tiles ||
+        (const char*)(M.tiles + l.tiles.size()) > (const char*)M.blocks || l.blocks.size() > room)
+        return hipErrorInvalidValue;
     auto up = [&](const void* dst, const void* src, size_t bytes) {
         return bytes ? hipMemcpyAsync(const_cast<void*>(dst), src, bytes, hipMemcpyHostToDevice, s) : hipSuccess;
     };
@@ -1245,7 +1255,8 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         mg_lists(B.hmg, B.mg_vols, &lists, &M);
         const size_t b_vols = align_up(sizeof(int) * lists.vols.size(), 256);
         const size_t b_tiles = align_up(sizeof(int2) * lists.tiles.size(), 256);
-        B.mg_list = dalloc(ctx, b_vols + b_tiles + sizeof(int2) * lists.blocks.size());
+        B.mg_room = nv == 1 ? lists.blocks.size() : mg_list_room(B.hmg, B.mg_vols);   // a batch's tail is listed anew
+        B.mg_list = dalloc(ctx, b_vols + b_tiles + sizeof(int2) * B.mg_room);
         if (!mem || !B.mg_list) return FAST_E_OOM;
         char* q = (char*)B.mg_list;
         M.vol = (const MgDesc*)(m + o_mg);
@@ -1255,7 +1266,7 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         M.tiles = (const int2*)(q + b_vols);
         M.blocks = (const int2*)(q + b_vols + b_tiles);
         if (e == hipSuccess) e = hipMemcpyAsync(m + o_mg, B.hmg.data(), sizeof(MgDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess) e = mg_upload(M, lists, ctx->stream);
+        if (e == hipSuccess) e = mg_upload(M, lists, B.mg_room, ctx->stream);
         if (e == hipSuccess) e = ft::mg_setup(L, M, ctx->stream);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);   // the copies read hrb, hmg and the lists
@@ -1335,7 +1346,7 @@ static int solve_mixed_rb(fast_ctx* ctx, std::vector<Job*>& jobs) {
                 if (snap[i].status != ST_IDLE) mv.push_back(i);
             MgLists lists;
             mg_lists(B.hmg, mv, &lists, &B.M);
-            if (e2 == hipSuccess) e2 = mg_upload(B.M, lists, s);
+            if (e2 == hipSuccess) e2 = mg_upload(B.M, lists, B.mg_room, s);
             if (e2 == hipSuccess) e2 = hipStreamSynchronize(s);   // the copies read the lists
         }
         drop_graph();
@@ -1695,6 +1706,28 @@ int fast_debug_stream(fast_ctx* ctx, size_t bytes, int iters, double* ms) {
     dfree(ctx, b);
     dfree(ctx, a);
     return rc;
+}
+
+int fast_debug_mg_lists(int n, const int* dims, const int* dirs, const uint8_t* live, uint64_t* blocks) {
+    if (n < 1 || !dims || !dirs || !live || !blocks) return FAST_E_BADARG;
+    std::vector<MgDesc> desc(n);
+    std::vector<int> all, part;
+    for (int i = 0; i < n; ++i) {
+        size_t floats = 0;
+        if (dims[3 * i] < 1 || dims[3 * i + 1] < 1 || dims[3 * i + 2] < 1 || dirs[i] < 0 || dirs[i] > 5) return FAST_E_BADARG;
+        if (!mg_plan(dims[3 * i], dims[3 * i + 1], dims[3 * i + 2], dirs[i] / 2, &desc[i], &floats)) continue;
+        all.push_back(i);
+        if (live[i]) part.push_back(i);
+    }
+    mg_tile(desc, all);
+    MgLists lists;
+    MgLaunch M{};
+    blocks[0] = mg_list_room(desc, all);
+    mg_lists(desc, all, &lists, &M);
+    blocks[1] = lists.blocks.size();
+    mg_lists(desc, part, &lists, &M);
+    blocks[2] = lists.blocks.size();
+    return FAST_OK;
 }
 
 int fast_debug_apply_f64(fast_volume* vol, int dir, const double* x, double* y) { return debug_apply<double>(vol, dir, x, y); }

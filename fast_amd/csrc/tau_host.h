@@ -148,7 +148,12 @@ struct MgLists {
     std::vector<int2> tiles, blocks;
 };
 void mg_lists(const std::vector<ft::MgDesc>& desc, const std::vector<int>& vols, MgLists* out, ft::MgLaunch* M);
-hipError_t mg_upload(const ft::MgLaunch& M, const MgLists& lists, hipStream_t s);
+// Blocks that the lists of `vols` or of any part of them can have.  A part may have more blocks than the
+// whole (fewer volumes take fewer planes per tile), but none more than at the fewest planes.
+size_t mg_list_room(const std::vector<ft::MgDesc>& desc, const std::vector<int>& vols);
+// The lists to where M points, vols then tiles then blocks in one device block with room for `room` blocks;
+// an error where they do not fit.
+hipError_t mg_upload(const ft::MgLaunch& M, const MgLists& lists, size_t room, hipStream_t s);
 // Form of the red-black Y and Q passes (RbLaunch::staged): FAST_TAU_RB_STAGED = 0 (separate,
 // Q reads six Y values), 1 (separate, Q stages the Y planes in LDS), default 2 (fused).
 int rb_mode();

@@ -295,7 +295,8 @@ struct MgLaunch {
 bool mg_plan(int nx, int ny, int nz, int primary, MgDesc* d, size_t* floats);
 // Splits the fine grids of the listed volumes, which run together, into tiles; returns their number.
 int mg_tile(std::vector<MgDesc>& d, const std::vector<int>& vols);
-// The same for one level of several volumes: planes per tile, tiles of a volume.
+// The same for one level of several volumes: planes per tile (at least kMgLeastTz), tiles of a volume.
+constexpr int kMgLeastTz = 2;
 int mg_level_tz(const std::vector<MgLevel>& l);
 int mg_level_tiles(const MgLevel& l, int tz);
 // Level coefficients and FP32 tables (codes and Coef uploaded before).

@@ -340,6 +340,11 @@ int fast_debug_time_passes(fast_volume* vol, int dir, int precision, int solver,
  * update, r.r, r.D^-1 r), each launched `iters` times back to back; ms[4] = mean period of a
  * whole iteration.  ms: 5 doubles. */
 int fast_debug_time_rb_passes(fast_volume* vol, int dir, int iters, double* ms);
+/* Launch lists of the multigrid preconditioner (host arithmetic only) for a batch of n volumes of extents
+ * dims[3 i ..] solved in direction dirs[i], live[i] != 0 for those that are still unfinished when the batch
+ * is compacted: blocks[0] = coarse-level blocks there is room for, blocks[1] = those of the whole batch,
+ * blocks[2] = those of the unfinished volumes. */
+int fast_debug_mg_lists(int n, const int* dims, const int* dirs, const uint8_t* live, uint64_t* blocks);
 /* Measured HBM ceiling: streaming kernels over three device buffers of `bytes` each (16-byte
  * accesses), each launched `iters` times back to back after one untimed launch (HIP events):
  * ms[0] c = a + s b with one float4 per thread, ms[1] the same on 8192 striding blocks,
