@@ -341,7 +341,7 @@ __device__ __forceinline__ void reduce_volume_wave(const double* part, int base,
 // CG.cpp:85-92; GPU mirrors fastlib/src/cuda/BICGSTAB.cu:93-213, CG.cu:68-155).
 // ---------------------------------------------------------------------------------------
 template <class A>
-__device__ __forceinline__ void bicg_loop_head(VolState<A>* s, A rr0) {
+__host__ __device__ __forceinline__ void bicg_loop_head(VolState<A>* s, A rr0) {
     // while (|r|^2 > tol2 && i < maxIters) { rho_old = rho; rho = r0.r; restart?; beta = ... }
     if (!(s->rsq > s->tol2) || s->iter >= s->maxiter) {
         s->status = ST_DONE;
@@ -369,8 +369,8 @@ __device__ __forceinline__ void bicg_loop_head(VolState<A>* s, A rr0) {
 // correction and starts afresh from x64.  BiCGSTAB's residual peaks by orders of magnitude
 // on ill-conditioned volumes and recovers, so growth alone drops nothing by default.
 template <class A>
-__device__ __forceinline__ void mixed_after_iteration(VolState<A>* s, A rr0) {
-    if (!isfinite(s->rsq) || s->rsq > s->blowup2 * s->rsq_ref) {
+__host__ __device__ __forceinline__ void mixed_after_iteration(VolState<A>* s, A rr0) {
+    if (!__builtin_isfinite(s->rsq) || s->rsq > s->blowup2 * s->rsq_ref) {
         s->status = ST_FRESH;
         s->discard = 1;
         return;
@@ -380,7 +380,7 @@ __device__ __forceinline__ void mixed_after_iteration(VolState<A>* s, A rr0) {
         s->rho_rec = rr0;
         return;
     }
-    if (!isfinite(rr0) || fabs(rr0) < s->eps2 * s->r0sq || fabs(rr0) < s->restart_cos * sqrt(s->r0sq * s->rsq)) {
+    if (!__builtin_isfinite(rr0) || fabs(rr0) < s->eps2 * s->r0sq || fabs(rr0) < s->restart_cos * sqrt(s->r0sq * s->rsq)) {
         s->status = ST_UPDATE;
         s->reshadow = 1;
         return;
@@ -395,14 +395,43 @@ __device__ __forceinline__ void mixed_after_iteration(VolState<A>* s, A rr0) {
     s->status = ST_RUNNING;
 }
 
+// A preconditioned volume goes on with the Jacobi form, starting afresh from its x64.  The iterations
+// count from 0 again (as at Eigen's first restart), so that the cap leaves the Jacobi form what
+// it had without the cycle.
+template <class A>
+__host__ __device__ __forceinline__ void mg_leave(VolState<A>* s) {
+    s->mg = 0;
+    s->iter = 0;
+    s->status = ST_FRESH;
+}
+
+// Breakdown of a mixed CG: a fresh start from x64.  The same cycle on the same residual would break down
+// again, so a preconditioned volume also leaves it.
+template <class A>
+__host__ __device__ __forceinline__ void cg_breakdown(VolState<A>* s) {
+    s->status = ST_FRESH;
+    if (s->mg) mg_leave(s);
+}
+
+// r.z of a preconditioned volume's cycle.  It is negative for every r, as D and A are, unless the cycle, in
+// FP32, has overflowed or is not definite here.
+__host__ __device__ __forceinline__ void mg_beta(VolState<double>* s, double rz) {
+    if (!(rz < 0.0) || !__builtin_isfinite(rz)) {
+        mg_leave(s);
+        return;
+    }
+    if (!s->first) s->beta = rz / s->absnew;
+    s->absnew = rz;
+}
+
 // Mixed form, CG: the same update / fresh-start rules; between updates the usual PCG
 // recurrence (beta = r.z / previous r.z).
 template <class A>
-__device__ __forceinline__ void mixed_cg_after_iteration(VolState<A>* s, A rz) {
+__host__ __device__ __forceinline__ void mixed_cg_after_iteration(VolState<A>* s, A rz) {
     s->iter += 1;
-    if (!isfinite(s->rsq) || s->rsq > 1e4 * s->rsq_ref) {
-        s->status = ST_FRESH;
+    if (!__builtin_isfinite(s->rsq) || s->rsq > 1e4 * s->rsq_ref) {
         s->discard = 1;
+        cg_breakdown(s);
         return;
     }
     if (!(s->rsq > s->tol2) || s->rsq < s->delta2 * s->rsq_ref || s->iter >= s->maxiter) {
@@ -410,8 +439,7 @@ __device__ __forceinline__ void mixed_cg_after_iteration(VolState<A>* s, A rz) {
         return;
     }
     if (s->mg && ++s->mg_since >= s->mg_stall) {
-        s->mg = 0;
-        s->status = ST_FRESH;
+        mg_leave(s);
         return;
     }
     s->first = 0;
@@ -425,7 +453,7 @@ __device__ __forceinline__ void mixed_cg_after_iteration(VolState<A>* s, A rz) {
 // Scalar update of one volume after a pass, from the pass's dot products `tot` (run by one
 // thread of the volume's last tile).
 template <class A, int KIND>
-__device__ void fin_update(VolState<A>* s, const A* tot) {
+__host__ __device__ void fin_update(VolState<A>* s, const A* tot) {
     switch (KIND) {
         case F_INIT_BICG: {
             s->rsq = tot[0];
@@ -456,12 +484,12 @@ __device__ void fin_update(VolState<A>* s, const A* tot) {
         }
         case F_BICG1:
             s->alpha = s->rho / tot[0];
-            if (s->mode == 1 && !isfinite(s->alpha)) s->status = ST_FRESH;   // breakdown: start afresh
+            if (s->mode == 1 && !__builtin_isfinite(s->alpha)) s->status = ST_FRESH;   // breakdown: start afresh
             break;
         case F_BICG2: {
             const A tmp = tot[1];
             s->omega = (tmp > A(0)) ? tot[0] / tmp : A(0);
-            if (s->mode == 1 && !isfinite(s->omega)) s->status = ST_FRESH;
+            if (s->mode == 1 && !__builtin_isfinite(s->omega)) s->status = ST_FRESH;
             break;
         }
         case F_BICG3: {
@@ -496,7 +524,7 @@ __device__ void fin_update(VolState<A>* s, const A* tot) {
         }
         case F_CG1:
             s->alpha = s->absnew / tot[0];
-            if (s->mode == 1 && !isfinite(s->alpha)) s->status = ST_FRESH;
+            if (s->mode == 1 && !__builtin_isfinite(s->alpha)) cg_breakdown(s);
             break;
         case F_CG2: {
             s->rsq = tot[0];
@@ -526,7 +554,7 @@ __device__ void fin_update(VolState<A>* s, const A* tot) {
 // Finalize of a reliable update / fresh start: the FP64 test decides whether the volume is
 // finished; otherwise BiCGSTAB continues on the replaced residual (a fresh start takes the
 // Eigen initial state with r0 = r).
-__device__ void mixres_update(VolState<double>* s, const double* tot) {
+__host__ __device__ void mixres_update(VolState<double>* s, const double* tot) {
     const int status = s->status;
     if (s->refinements == 0) {
         s->b64sq = tot[1];
@@ -568,9 +596,9 @@ __device__ void mixres_update(VolState<double>* s, const double* tot) {
     }
     if (status == ST_FRESH || reshadow) s->r0sq = tot[2];
     if (reshadow && status != ST_FRESH) s->restarts += 1;
-    const double rho_new = (status != ST_FRESH && !reshadow && isfinite(s->rho_rec)) ? s->rho_rec : tot[3];
+    const double rho_new = (status != ST_FRESH && !reshadow && __builtin_isfinite(s->rho_rec)) ? s->rho_rec : tot[3];
     if (status != ST_FRESH && !reshadow &&
-        (!isfinite(rho_new) || fabs(rho_new) < s->restart_cos * sqrt(s->r0sq * s->rsq))) {
+        (!__builtin_isfinite(rho_new) || fabs(rho_new) < s->restart_cos * sqrt(s->r0sq * s->rsq))) {
         s->status = ST_UPDATE;   // the replaced residual is too orthogonal to r0: reset r0 next
         s->reshadow = 1;
         return;

@@ -652,7 +652,8 @@ __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLa
     for (int i = tid; i < sl[b].n; i += kMgBottomThreads) mem[off_b + (unsigned)sl[b].n + i] = u[i];
 }
 
-// r.z of one preconditioned volume, then beta = r.z / (previous r.z).
+// r.z of one preconditioned volume, then beta = r.z / (previous r.z).  Where mg_beta ends the cycle the passes of
+// this iteration leave the volume alone; x's pending step is in the buffer the cycle did not write.
 __global__ __launch_bounds__(kFinThreads) void k_mg_fin(RbLaunch L, MgLaunch M) {
     const int v = L.solo ? 0 : M.vols[blockIdx.x];
     VolState<double>* s = L.st + v;
@@ -667,11 +668,7 @@ __global__ __launch_bounds__(kFinThreads) void k_mg_fin(RbLaunch L, MgLaunch M) 
     }
     __shared__ double red[2];
     block_reduce_store<AccDD, 1, kFinThreads>(sum, red);
-    if (threadIdx.x == 0) {
-        const double rz = red[0] + red[1];
-        if (!s->first) s->beta = rz / s->absnew;
-        s->absnew = rz;
-    }
+    if (threadIdx.x == 0) mg_beta(s, red[0] + red[1]);
 }
 
 // ---- set-up --------------------------------------------------------------------------------
@@ -996,6 +993,20 @@ int mg_tile(std::vector<MgDesc>& d, const std::vector<int>& vols) {
         tiles += m.ntiles;
     }
     return tiles;
+}
+
+void cg_state_event(VolState<double>* s, int event, double value) {
+    const bool update = s->status == ST_UPDATE || s->status == ST_FRESH;
+    if (event == 0 ? !update : s->status != ST_RUNNING) return;
+    const double tot[4] = {value, event == 0 ? 1.0 : -value, value, -value};
+    if (event == 0)
+        mixres_update(s, tot);
+    else if (event == 1 && s->mg)
+        mg_beta(s, value);
+    else if (event == 2)
+        fin_update<double, F_CG1>(s, tot);
+    else if (event == 3)
+        fin_update<double, F_CG2>(s, tot);
 }
 
 hipError_t mg_setup(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {

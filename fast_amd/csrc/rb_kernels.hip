@@ -221,7 +221,7 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
         if (tile == d.tile_base && threadIdx.x == 0) {
             vs->alpha = alpha;
             if (vs->xpend == (mg ? 1 : 2)) vs->xpend = 0;   // the P pass of this iteration added them
-            if (!isfinite(alpha)) vs->status = ST_FRESH;
+            if (!isfinite(alpha)) cg_breakdown(vs);
         }
         if (!isfinite(alpha)) return;
     }

@@ -1730,6 +1730,26 @@ int fast_debug_mg_lists(int n, const int* dims, const int* dirs, const uint8_t* 
     return FAST_OK;
 }
 
+int fast_debug_cg_state(int mg, double tolerance, long max_iter, int n, const int* events, const double* values,
+                        int64_t* out) {
+    if (n < 0 || !events || !values || !out) return FAST_E_BADARG;
+    VolState<double> s{};
+    s.status = ST_FRESH;
+    s.mode = 1;
+    s.solver = FAST_CG;
+    s.tol = s.otol = tolerance;
+    s.maxiter = max_iter;
+    s.delta2 = 0.01;
+    s.mg = mg ? 1 : 0;
+    s.mg_stall = kMgStall;
+    for (int i = 0; i < n; ++i) {
+        cg_state_event(&s, events[i], values[i]);
+        const int64_t now[4] = {s.status, s.mg, s.iter, s.refinements};
+        std::memcpy(out + 4 * i, now, sizeof(now));
+    }
+    return FAST_OK;
+}
+
 int fast_debug_apply_f64(fast_volume* vol, int dir, const double* x, double* y) { return debug_apply<double>(vol, dir, x, y); }
 int fast_debug_apply_f32(fast_volume* vol, int dir, const float* x, float* y) { return debug_apply<float>(vol, dir, x, y); }
 

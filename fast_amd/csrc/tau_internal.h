@@ -248,7 +248,8 @@ inline int rb_row_pitch(int hx) { return (hx + 2 + 3) & ~3; }
 // two sweeps give z = D_r^-1 (r + A_rb Y(x2)).  None of these sums cancels, so the cycle runs in
 // FP32; the CG around it keeps its FP64 arithmetic, FP64 residuals and stopping rule.
 // A volume whose residual has not dropped to its next reliable update within kMgStall iterations
-// (seen at solid conductivities of 1e-6 and 95% solid) goes on with the Jacobi form from its x64.
+// (seen at solid conductivities of 1e-6 and 95% solid), or has grown 100-fold since the last one, or
+// whose r.z or p.q break down, goes on with the Jacobi form from its x64.
 // The last level has at most 64 cells and is solved with its inverse.  Level l >= 1 holds, per cell, the right-hand side (overwritten by the solution), the black
 // values of the first sweep, the face coefficients towards x+, y+ and z+, and 1 / diagonal, all
 // for -A (positive).  Levels from `bottom` on are solved by one block per volume in LDS.
@@ -303,6 +304,11 @@ int mg_level_tiles(const MgLevel& l, int tz);
 hipError_t mg_setup(const RbLaunch&, const MgLaunch&, hipStream_t);
 // z = B r into the buffer of the next p, then beta, for the running volumes that are preconditioned.
 hipError_t mg_cycle(const RbLaunch&, const MgLaunch&, hipStream_t);
+
+// One scalar update of a red-black CG, as the kernels apply it to a volume in that status (host; for tests):
+// 0 reliable update with |r|^2 = value (|b|^2 = 1), 1 cycle with r.z = value, 2 p.q = value, 3 |r|^2 = value
+// and r.z = -value at the end of an iteration.
+void cg_state_event(VolState<double>* s, int event, double value);
 
 // Diagonal tables and per-colour codes (after the vectors and codes were zero-filled).
 hipError_t rb_setup(const RbLaunch&, hipStream_t);

@@ -86,7 +86,8 @@ typedef struct fast_tau_result {
     double dc;            /* mean boundary flux (VolumeMeasures.cpp:274) */
     double rel_residual;  /* solver error: sqrt(|r|^2/|b|^2) of the recursive residual */
     double true_rel_residual; /* MIXED: FP64 true residual at exit; otherwise -1 */
-    long iterations;      /* Krylov iterations */
+    long iterations;      /* Krylov iterations (MIXED: where a solve gave up the multigrid preconditioner, those
+                             since then) */
     int status;           /* fast_status */
     int restarts;         /* BiCGSTAB restarts (rho breakdown; MIXED: fresh starts) */
     int refinements;      /* MIXED: FP64 true-residual replacements (reliable updates) */
@@ -345,6 +346,12 @@ int fast_debug_time_rb_passes(fast_volume* vol, int dir, int iters, double* ms);
  * is compacted: blocks[0] = coarse-level blocks there is room for, blocks[1] = those of the whole batch,
  * blocks[2] = those of the unfinished volumes. */
 int fast_debug_mg_lists(int n, const int* dims, const int* dirs, const uint8_t* live, uint64_t* blocks);
+/* The scalar recurrence of one mixed CG volume (host arithmetic only), multigrid-preconditioned if mg, through n
+ * events: 0 a reliable update that finds |r|^2 = values[i] (|b|^2 = 1), 1 a multigrid cycle with r.z = values[i],
+ * 2 p.q = values[i], 3 the end of an iteration with |r|^2 = -r.D^-1 r = values[i] (D is negative).  Events that do not fit the
+ * status are passed over, as the kernels do.  out: {status, mg, iterations, updates} after each event. */
+int fast_debug_cg_state(int mg, double tolerance, long max_iter, int n, const int* events, const double* values,
+                        int64_t* out);
 /* Measured HBM ceiling: streaming kernels over three device buffers of `bytes` each (16-byte
  * accesses), each launched `iters` times back to back after one untimed launch (HIP events):
  * ms[0] c = a + s b with one float4 per thread, ms[1] the same on 8192 striding blocks,
