@@ -210,7 +210,18 @@ __device__ __forceinline__ void wave_combine(Acc& a) {
     }
 }
 
-// Deterministic block reduction of NP accumulators; thread 0 writes out[2k], out[2k+1].
+// Between the lanes of one wave that write LDS (or memory) and other lanes of it that read it: no instruction of
+// its own, since a wave's LDS accesses are carried out in order, but the compiler keeps that order.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// 32-bit words of an object of any type, for copying it by the lanes of a block.
+typedef unsigned __attribute__((may_alias)) alias_word;
+
+// Deterministic block reduction of NP accumulators; lane 16 k of the first wave writes out[2k], out[2k+1].
 template <class Acc, int NP, int NT>
 __device__ __forceinline__ void block_reduce_store(Acc (&acc)[NP], double* out) {
     constexpr int NW = NT / 64;
@@ -297,7 +308,8 @@ __device__ __forceinline__ void reduce_volume(const double* part, int base, int 
 #pragma unroll
             for (int k = 0; k < NP; ++k) sums[k].add2(v[u][2 * k], v[u][2 * k + 1]);
     }
-    block_reduce_store<AccDD, NP, NT>(sums, red);   // written by the first wave, read by it
+    block_reduce_store<AccDD, NP, NT>(sums, red);
+    wave_sync();   // written by lanes of the first wave, read by its first
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int k = 0; k < NP; ++k) tot[k] = red[2 * k] + red[2 * k + 1];

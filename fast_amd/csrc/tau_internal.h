@@ -156,7 +156,8 @@ struct Passes {
     // Same, recording ev[2k] / ev[2k+1] around stencil pass k (k = 0, 1).
     static hipError_t cg_iter_timed(const Launch<T, A>&, hipStream_t, hipEvent_t* ev);
     // `iters` iterations with the finalizes inside the next pass (T = A only): one launch per pass
-    // and one per round, where cg_iter and bicg_iter take two per pass.  Same results bit for bit.
+    // and one per round, where cg_iter and bicg_iter take two per pass.  The same sums in another order: the same
+    // bits but where a sum is within about 2^-104 of a rounding tie.
     static hipError_t round_folded(const Launch<T, A>&, int solver, int iters, hipStream_t);
     // Stencil kernel of pass k alone (k = 0, 1 for CG; 0, 1, 2 for BiCGSTAB), no finalize
     // (timing: the volumes' scalars and statuses stay as they are).

@@ -580,8 +580,9 @@ __host__ __device__ constexpr int np_of(int fin) {
 
 // FOLD: the finalize of the previous pass (FinKind), run here instead of in a launch of its own.
 // Every block of a volume reduces that pass's partials and updates a copy of the volume's
-// scalars in LDS while its first planes load: a double-double sum rounds to the same value in
-// any order, so all blocks and k_fin agree to the last bit.  The block of the first tile stores the
+// scalars in LDS while its first planes load.  All blocks add in the same order and agree to the last bit;
+// k_fin's order is another, whose double-double sum differs by about 2^-104 and so rounds to the
+// same double unless the sum lies that close to a tie.  The block of the first tile stores the
 // state to the other of two buffers (blocks that start later still read the old one), and the
 // passes write their partials to alternating slots for the same reason.
 // A finalize launch costs 3.5-4.5 us and a gap on MI355X, the reduction by one wave about 1 us of a
@@ -611,8 +612,8 @@ __global__ __launch_bounds__(TX* TY) void k_stencil(Launch<T, A> L, const T* xin
     __shared__ VolState<A> sst;
     constexpr int SW = sizeof(VolState<A>) / 4;
     static_assert(SW <= 256 && sizeof(VolState<A>) % 4 == 0, "one word per thread");
-    const unsigned* st_w = reinterpret_cast<const unsigned*>(st);
-    unsigned* out_w = reinterpret_cast<unsigned*>(L.st_out + v);
+    const alias_word* st_w = reinterpret_cast<const alias_word*>(st);
+    alias_word* out_w = reinterpret_cast<alias_word*>(L.st_out + v);
     if (KIND != K_APPLY && KIND != K_RESTART && st->status != ST_RUNNING) {
         if (FOLD >= 0 && tile == vd.tile_base && (int)threadIdx.x < SW) out_w[threadIdx.x] = st_w[threadIdx.x];
         return;
@@ -666,11 +667,12 @@ __global__ __launch_bounds__(TX* TY) void k_stencil(Launch<T, A> L, const T* xin
         load_tables<C, TX * TY>(L.tab + (long long)v * 2 * kTabEntries, tab, ftab, pc.c);
         if constexpr (FOLD >= 0) {
             constexpr int NPF = np_of(FOLD);
-            // state and sums by the first wave, in order: no barrier before the update
+            // state and sums by the first wave: no barrier before the update
             if (threadIdx.x < 64)
-                for (int i = (int)threadIdx.x; i < SW; i += 64) reinterpret_cast<unsigned*>(&sst)[i] = st_w[i];
+                for (int i = (int)threadIdx.x; i < SW; i += 64) reinterpret_cast<alias_word*>(&sst)[i] = st_w[i];
             double tot[NPF];
             reduce_volume_wave<NPF>(L.part + (L.slot ^ 4), vd.tile_base, vd.ntiles, tot);
+            wave_sync();   // sst: written by all lanes of the wave, updated by its first
             if (threadIdx.x == 0) {
                 A ta[3] = {A(0), A(0), A(0)};
 #pragma unroll
@@ -679,7 +681,7 @@ __global__ __launch_bounds__(TX* TY) void k_stencil(Launch<T, A> L, const T* xin
             }
             __syncthreads();
             if (tile == vd.tile_base && (int)threadIdx.x < SW)
-                out_w[threadIdx.x] = reinterpret_cast<const unsigned*>(&sst)[threadIdx.x];
+                out_w[threadIdx.x] = reinterpret_cast<const alias_word*>(&sst)[threadIdx.x];
             pc.first = sst.first;
             pc.alpha = C(sst.alpha);
             pc.beta = C(sst.beta);
@@ -735,7 +737,7 @@ __global__ __launch_bounds__(kFinThreads) void k_fin(Launch<T, A> L) {
     if (L.st_out != L.st) {   // end of a folded round: the state moves back to its first buffer
         constexpr int SW = sizeof(VolState<A>) / 4;
         if ((int)threadIdx.x < SW)
-            reinterpret_cast<unsigned*>(L.st_out + v)[threadIdx.x] = reinterpret_cast<const unsigned*>(s)[threadIdx.x];
+            reinterpret_cast<alias_word*>(L.st_out + v)[threadIdx.x] = reinterpret_cast<const alias_word*>(s)[threadIdx.x];
         s = L.st_out + v;
         __syncthreads();
     }
