@@ -176,27 +176,25 @@ static bool shape_compiled(int tx, int ty) {
 // against sweeps of all shapes: within 3-4% of the best on average and 10% at most, where one
 // shape per power-of-two size class was up to 2.3x off (FP64 CG, an iteration: 160x150x140 148 -> 63
 // us, 191x205x177 168 -> 108, 100^3 53 -> 41, 256^3 243 both).
-static Shape model_shape(const std::vector<const fast_volume*>& vols, int precision) {
+static Shape model_shape(const std::vector<std::array<int, 3>>& grids, int precision) {
     static const int kBySize[][2] = {{64, 16}, {64, 8}, {32, 32}, {32, 16}, {64, 4}, {32, 8}, {16, 16}};
     static const int k64x8[][2] = {{64, 8}, {64, 16}, {32, 16}, {32, 32}, {64, 4}, {32, 8}, {16, 16}};
     const bool fp64 = precision == FAST_FP64;
     const int held = precision == FAST_FP32 ? 24 : 16, prologue = fp64 ? 1 : 2;
     const double keeps_up = fp64 ? 12.0 : 18.0;   // waves on a CU beyond which a plane takes longer
     int nzmax = 1;
-    for (const fast_volume* v : vols) nzmax = std::max(nzmax, v->nz);
+    for (const auto& v : grids) nzmax = std::max(nzmax, v[2]);
     Shape best{64, 8, 16};
     double least = HUGE_VAL;
     for (const auto& s : fp64 ? kBySize : k64x8) {
         const int waves = s[0] * s[1] / 64;
         const long long cap = 256 * (held / waves);
-        int last = 0;
-        for (int n = 1; n <= nzmax; ++n) {   // tiles along z of the deepest volume
-            const int tz = (nzmax + n - 1) / n;
-            if (tz == last || tz > 64 || (tz < 2 && nzmax > 1)) continue;
-            last = tz;
+        for (int tz = std::min(64, nzmax); tz >= std::min(2, nzmax); --tz) {
+            const int n = (nzmax + tz - 1) / tz;   // tiles along z of the deepest volume
+            if ((nzmax + n - 1) / n != tz) continue;   // fewer planes make as many tiles
             long long tiles = 0;
-            for (const fast_volume* v : vols)
-                tiles += (long long)((v->nx + s[0] - 1) / s[0]) * ((v->ny + s[1] - 1) / s[1]) * ((v->nz + tz - 1) / tz);
+            for (const auto& v : grids)
+                tiles += (long long)((v[0] + s[0] - 1) / s[0]) * ((v[1] + s[1] - 1) / s[1]) * ((v[2] + tz - 1) / tz);
             auto plane = [&](long long blocks) { return std::max(1.0, (double)(blocks * waves) / keeps_up); };
             const long long rest = tiles % cap;
             const double t = (tz + prologue) *
@@ -216,7 +214,10 @@ Shape choose_shape(const std::vector<const fast_volume*>& vols, int precision, c
     for (const fast_volume* v : vols)
         if ((size_t)v->nx * v->ny * v->nz > (size_t)big->nx * big->ny * big->nz) big = v;
     auto it = ctx->tuned.find(shape_key(big->nx, big->ny, big->nz, precision));
-    return it != ctx->tuned.end() ? it->second : model_shape(vols, precision);
+    if (it != ctx->tuned.end()) return it->second;
+    std::vector<std::array<int, 3>> grids;
+    for (const fast_volume* v : vols) grids.push_back({v->nx, v->ny, v->nz});
+    return model_shape(grids, precision);
 }
 
 // Tuned tile shapes: text lines "<size-class key> <tx> <ty> <tz>" written by the autotuner
@@ -1706,6 +1707,20 @@ int fast_debug_stream(fast_ctx* ctx, size_t bytes, int iters, double* ms) {
     dfree(ctx, b);
     dfree(ctx, a);
     return rc;
+}
+
+int fast_debug_tile_shape(int n, const int* dims, int precision, int* shape) {
+    if (n < 1 || !dims || !shape || precision < FAST_FP64 || precision > FAST_MIXED) return FAST_E_BADARG;
+    std::vector<std::array<int, 3>> grids;
+    for (int i = 0; i < n; ++i) {
+        if (dims[3 * i] < 1 || dims[3 * i + 1] < 1 || dims[3 * i + 2] < 1) return FAST_E_BADARG;
+        grids.push_back({dims[3 * i], dims[3 * i + 1], dims[3 * i + 2]});
+    }
+    const Shape s = model_shape(grids, precision);
+    shape[0] = s.tx;
+    shape[1] = s.ty;
+    shape[2] = s.tz;
+    return FAST_OK;
 }
 
 int fast_debug_mg_lists(int n, const int* dims, const int* dirs, const uint8_t* live, uint64_t* blocks) {

@@ -1,0 +1,65 @@
+"""Tile shapes of the full-grid passes, on the CPU: the rule against a plain restatement, and its time on
+volumes that are very long in z."""
+import ctypes as C
+import time
+
+import numpy as np
+import pytest
+
+from fast_amd import _lib
+
+FP64, FP32, MIXED = 0, 1, 2
+
+
+def shape(dims, precision):
+    dims = np.ascontiguousarray(dims, np.int32)
+    out = (C.c_int * 3)()
+    assert _lib.lib().fast_debug_tile_shape(len(dims), dims.ctypes.data_as(C.POINTER(C.c_int)), precision, out) == 0
+    return tuple(out)
+
+
+def up(a, b):
+    return -(-a // b)
+
+
+def plain(dims, precision):
+    """The least modelled time over every number of tiles along z."""
+    order = ([(64, 16), (64, 8), (32, 32), (32, 16), (64, 4), (32, 8), (16, 16)] if precision == FP64 else
+             [(64, 8), (64, 16), (32, 16), (32, 32), (64, 4), (32, 8), (16, 16)])
+    held, prologue, keeps_up = (24 if precision == FP32 else 16), (1 if precision == FP64 else 2), (12 if precision == FP64 else 18)
+    nz = max(d[2] for d in dims)
+    best = None
+    for tx, ty in order:
+        waves = tx * ty // 64
+        cap, last = 256 * (held // waves), 0
+        for n in range(1, nz + 1):
+            tz = up(nz, n)
+            if tz == last or tz > 64 or (tz < 2 and nz > 1):
+                continue
+            last = tz
+            tiles = sum(up(x, tx) * up(y, ty) * up(z, tz) for x, y, z in dims)
+            full, rest = divmod(tiles, cap)
+            t = (tz + prologue) * (full * max(1.0, held // waves * waves / keeps_up) +
+                                   (max(1.0, up(rest, 256) * waves / keeps_up) if rest else 0.0))
+            if best is None or t < best[0]:
+                best = (t, (tx, ty, tz))
+    return best[1]
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32, MIXED])
+def test_the_rule_is_the_plain_one(precision):
+    rng = np.random.default_rng(precision)
+    for _ in range(60):
+        d = [tuple(int(v) for v in np.exp(rng.uniform(0, np.log(400), 3)).round())]
+        assert shape(d, precision) == plain(d, precision), d
+    assert shape([(1, 1, 1)], precision)[2] == 1
+
+
+def test_long_volumes_take_no_time():
+    """2^29 voxels, all along z, are chosen for in well under a millisecond of host time per call (a loop
+    over the tiles along z took seconds)."""
+    t = time.perf_counter()
+    for _ in range(10):
+        s = shape([(1, 1, (1 << 29) - 1)], FP64)
+    assert time.perf_counter() - t < 0.1
+    assert 2 <= s[2] <= 64
