@@ -176,9 +176,19 @@ static bool shape_compiled(int tx, int ty) {
 // against sweeps of all shapes: within 3-4% of the best on average and 10% at most, where one
 // shape per power-of-two size class was up to 2.3x off (FP64 CG, an iteration: 160x150x140 148 -> 63
 // us, 191x205x177 168 -> 108, 100^3 53 -> 41, 256^3 243 both).
-static Shape model_shape(const std::vector<std::array<int, 3>>& grids, int precision) {
-    static const int kBySize[][2] = {{64, 16}, {64, 8}, {32, 32}, {32, 16}, {64, 4}, {32, 8}, {16, 16}};
-    static const int k64x8[][2] = {{64, 8}, {64, 16}, {32, 16}, {32, 32}, {64, 4}, {32, 8}, {16, 16}};
+//
+// Where a batch runs more than two rounds the vectors' traffic counts, which the model does not hold:
+// narrow blocks read more halo, and idle lanes past a row's end cost none.  There the choice is
+// among 64x8, 64x4 and 32x8 (taken as 10% slower).  Against the choice among all shapes, mostly 16x16: 10 volumes of 100 to
+// 160 edge, FP32 CG 19.9 -> 17.1 ms, FP64 32.5 -> 31.4; 4 of 150 to 200 edge 14.8 -> 13.0 and 26.9 -> 23.4.
+struct BlockShape {
+    int tx, ty;
+    double weight;   // of a round's time
+};
+
+template <int N>
+static Shape least_time(const std::vector<std::array<int, 3>>& grids, int precision, const BlockShape (&shapes)[N],
+                        double* rounds) {
     const bool fp64 = precision == FAST_FP64;
     const int held = precision == FAST_FP32 ? 24 : 16, prologue = fp64 ? 1 : 2;
     const double keeps_up = fp64 ? 12.0 : 18.0;   // waves on a CU beyond which a plane takes longer
@@ -186,26 +196,39 @@ static Shape model_shape(const std::vector<std::array<int, 3>>& grids, int preci
     for (const auto& v : grids) nzmax = std::max(nzmax, v[2]);
     Shape best{64, 8, 16};
     double least = HUGE_VAL;
-    for (const auto& s : fp64 ? kBySize : k64x8) {
-        const int waves = s[0] * s[1] / 64;
+    for (const BlockShape& s : shapes) {
+        const int waves = s.tx * s.ty / 64;
         const long long cap = 256 * (held / waves);
         for (int tz = std::min(64, nzmax); tz >= std::min(2, nzmax); --tz) {
             const int n = (nzmax + tz - 1) / tz;   // tiles along z of the deepest volume
             if ((nzmax + n - 1) / n != tz) continue;   // fewer planes make as many tiles
             long long tiles = 0;
             for (const auto& v : grids)
-                tiles += (long long)((v[0] + s[0] - 1) / s[0]) * ((v[1] + s[1] - 1) / s[1]) * ((v[2] + tz - 1) / tz);
+                tiles += (long long)((v[0] + s.tx - 1) / s.tx) * ((v[1] + s.ty - 1) / s.ty) * ((v[2] + tz - 1) / tz);
             auto plane = [&](long long blocks) { return std::max(1.0, (double)(blocks * waves) / keeps_up); };
             const long long rest = tiles % cap;
-            const double t = (tz + prologue) *
+            const double t = (tz + prologue) * s.weight *
                              ((double)(tiles / cap) * plane(held / waves) + (rest ? plane((rest + 255) / 256) : 0.0));
             if (t < least) {
                 least = t;
-                best = Shape{s[0], s[1], tz};
+                best = Shape{s.tx, s.ty, tz};
+                *rounds = (double)tiles / (double)cap;
             }
         }
     }
     return best;
+}
+
+static Shape model_shape(const std::vector<std::array<int, 3>>& grids, int precision) {
+    static const BlockShape kBySize[] = {{64, 16, 1.0}, {64, 8, 1.0}, {32, 32, 1.0}, {32, 16, 1.0},
+                                         {64, 4, 1.0},  {32, 8, 1.0}, {16, 16, 1.0}};
+    static const BlockShape k64x8[] = {{64, 8, 1.0}, {64, 16, 1.0}, {32, 16, 1.0}, {32, 32, 1.0},
+                                       {64, 4, 1.0}, {32, 8, 1.0},  {16, 16, 1.0}};
+    static const BlockShape kManyRounds[] = {{64, 8, 1.0}, {64, 4, 1.0}, {32, 8, 1.1}};
+    double rounds = 0;
+    const Shape s = precision == FAST_FP64 ? least_time(grids, precision, kBySize, &rounds)
+                                           : least_time(grids, precision, k64x8, &rounds);
+    return grids.size() > 1 && rounds > 2.0 ? least_time(grids, precision, kManyRounds, &rounds) : s;
 }
 
 Shape choose_shape(const std::vector<const fast_volume*>& vols, int precision, const fast_ctx* ctx) {
