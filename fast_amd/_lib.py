@@ -147,6 +147,7 @@ PROTOTYPES = [
     ("fast_debug_system_f64", C.c_int, [_vp, C.c_int, _dp, _dp, _dp]),
     ("fast_debug_time_passes", C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, _dp]),
     ("fast_debug_time_rb_passes", C.c_int, [_vp, C.c_int, C.c_int, _dp]),
+    ("fast_debug_folds", C.c_int, [C.c_int, C.POINTER(C.c_int), C.c_int]),
     ("fast_debug_tile_shape", C.c_int, [C.c_int, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int)]),
     ("fast_debug_mg_lists", C.c_int, [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), _u8p, C.POINTER(C.c_uint64)]),
     ("fast_debug_cg_state", C.c_int, [C.c_int, C.c_double, C.c_long, C.c_int, C.POINTER(C.c_int), _dp, C.POINTER(C.c_int64)]),

@@ -21,6 +21,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <numeric>
 #include <string>
 #include <unordered_map>
 #include <tuple>
@@ -866,6 +867,11 @@ static int finish(BT& B, const VolDesc* vol_dev, const TC* conc, const Coef<TC>*
     return FAST_OK;
 }
 
+// Whether the passes of a plain solve run the finalizes themselves (kFoldMaxTiles*).
+static bool folds_finalizes(int most, int total, bool fp64) {
+    return most <= (fp64 ? kFoldMaxTilesF64 : kFoldMaxTilesF32) && total <= kFoldMaxTilesBatch;
+}
+
 template <class T, class A>
 static int solve_plain(fast_ctx* ctx, std::vector<Job*>& jobs, Shape shape, int solver) {
     Batch<T, A> B;
@@ -884,7 +890,7 @@ static int solve_plain(fast_ctx* ctx, std::vector<Job*>& jobs, Shape shape, int 
     const long max_chunks = 3 * (maxit / chunk + 2) + 16;
     int most = 0;
     for (const VolDesc& d : B.hvol) most = std::max(most, d.ntiles);
-    const bool fold = most <= (sizeof(T) == 8 ? kFoldMaxTilesF64 : kFoldMaxTilesF32);
+    const bool fold = folds_finalizes(most, B.L.ntiles, sizeof(T) == 8);
     auto round = [&]() -> hipError_t {
         if (fold) return Passes<T, A>::round_folded(B.L, solver, chunk, s);
         for (int i = 0; i < chunk; ++i) {
@@ -1730,6 +1736,11 @@ int fast_debug_stream(fast_ctx* ctx, size_t bytes, int iters, double* ms) {
     dfree(ctx, b);
     dfree(ctx, a);
     return rc;
+}
+
+int fast_debug_folds(int n, const int* tiles, int precision) {
+    if (n < 1 || !tiles) return 0;
+    return folds_finalizes(*std::max_element(tiles, tiles + n), std::accumulate(tiles, tiles + n, 0), precision == FAST_FP64);
 }
 
 int fast_debug_tile_shape(int n, const int* dims, int precision, int* shape) {

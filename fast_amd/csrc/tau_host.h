@@ -31,7 +31,11 @@ constexpr int kRbCompactMin = 512;
 // 64^3 (256 tiles) 18.2 / 29.0 and 21.2 / 33.1 us, 100^3 (1000 tiles) 34.9 / 57.3 and 36.5 / 60.1,
 // 256^3 (256) 226 / 428 and 231 / 435; FP32 64^3 16.4 and 18.8, 256^3 (768 tiles, three blocks per CU
 // with 58 registers) 141 and 122.
-constexpr int kFoldMaxTilesF64 = 1100, kFoldMaxTilesF32 = 512;
+// With more than about two rounds of blocks in all, a batch has the finalize launches' few us spread over a
+// long pass, and the reduction at every block's start and the registers cost more: 2971 tiles (16 volumes of 40 to 120
+// edge), each volume at most 324, FP32 CG 22.9 ms with and 21.1 without, FP64 33.2 and 31.1; but 1265 tiles
+// 12.3 and 13.1, 760 tiles FP64 17.4 and 18.9.
+constexpr int kFoldMaxTilesF64 = 1100, kFoldMaxTilesF32 = 512, kFoldMaxTilesBatch = 2048;
 // A one-volume red-black launch set of at most this many tiles has its U blocks reduce the
 // Q pass's partials into alpha themselves instead of a finalize launch: the blocks then fit
 // about one dispatch round, so the reduction at their start costs less than the launch it

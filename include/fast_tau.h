@@ -341,6 +341,9 @@ int fast_debug_time_passes(fast_volume* vol, int dir, int precision, int solver,
  * update, r.r, r.D^-1 r), each launched `iters` times back to back; ms[4] = mean period of a
  * whole iteration.  ms: 5 doubles. */
 int fast_debug_time_rb_passes(fast_volume* vol, int dir, int iters, double* ms);
+/* Whether FP64 or FP32 volumes of `tiles[i]` tiles solved together run each finalize inside the next pass (1) or as a
+ * launch of its own (0). */
+int fast_debug_folds(int n, const int* tiles, int precision);
 /* Tile shape (tx, ty, planes) that the full-grid passes take for a solve of n volumes of extents dims[3 i ..]
  * together, where neither fast_ctx_set_tile_shape nor a tuning line sets one (host arithmetic only). */
 int fast_debug_tile_shape(int n, const int* dims, int precision, int* shape);

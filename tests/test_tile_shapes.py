@@ -79,3 +79,15 @@ def test_long_volumes_take_no_time():
         s = shape([(1, 1, (1 << 29) - 1)], FP64)
     assert time.perf_counter() - t < 0.1
     assert 2 <= s[2] <= 64
+
+
+def test_large_batches_have_finalize_launches():
+    """A volume's finalizes are folded up to its tile limit, and a batch's only up to 2048 tiles in all."""
+    def folds(tiles, precision):
+        return _lib.lib().fast_debug_folds(len(tiles), (C.c_int * len(tiles))(*tiles), precision)
+
+    assert [folds([n], FP64) for n in (1, 1100, 1101)] == [1, 1, 0]
+    assert [folds([n], FP32) for n in (1, 512, 513)] == [1, 1, 0]
+    for precision in (FP64, FP32):
+        assert folds([256] * 8, precision) == 1 and folds([256] * 8 + [1], precision) == 0
+        assert folds([324] * 9 + [55], precision) == 0
