@@ -1003,16 +1003,15 @@ struct RbBatch {
     std::vector<MgDesc> hmg;     // by volume (nlev = 0: Jacobi)
     std::vector<int> mg_vols;    // preconditioned volumes
     MgLaunch M{};
-    void* mg_list = nullptr;     // launch lists on the device
-    size_t mg_room = 0;          // blocks that fit there
-    void* mg_mem = nullptr;      // level storage where the Y vector is in use (separate Y and Q passes)
+    void* mg_mem = nullptr;      // its descriptors, partials, tables and launch lists, and the level storage where
+                                 // the Y vector is in use (separate Y and Q passes)
+    size_t mg_room = 0;          // blocks that fit into the lists
 
     ~RbBatch() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (ctx) {
             dfree(ctx, meta);
             dfree(ctx, vecs);
-            dfree(ctx, mg_list);
             dfree(ctx, mg_mem);
         }
     }
@@ -1160,7 +1159,6 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
             B.mg_vols.push_back(i);
         }
     }
-    const int mg_tiles = mg_tile(B.hmg, B.mg_vols);
     B.ntiles = tiles;
     B.nplanes = planes;
     B.htile.resize(tiles);
@@ -1202,12 +1200,6 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
     o = align_up(o + sizeof(double) * planes, 256);
     const size_t o_tab = o;
     o = align_up(o + sizeof(double) * 2 * kTabEntries * nv, 256);
-    const size_t o_mg = o;
-    o = align_up(o + sizeof(MgDesc) * nv, 256);
-    const size_t o_mgpart = o;
-    o = align_up(o + sizeof(double) * 2 * (size_t)mg_tiles, 256);
-    const size_t o_mgtab = o;
-    o = align_up(o + sizeof(float) * kTabEntries * (mg_tiles ? nv : 0), 256);
     const size_t meta_bytes = o;
     // FP32 red vectors x, r, p[2], q (their region later holds the full-grid solution), then
     // FP64 y (black), x64 (red), x64b (black), then the per-colour codes
@@ -1217,6 +1209,36 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
     B.meta = dalloc(ctx, meta_bytes);
     B.vecs = dalloc(ctx, vec_bytes);
     if (!B.meta || !B.vecs) return FAST_E_OOM;
+    // What the preconditioner needs beside these is allocated last, in one block; where the budget has no room for it
+    // the batch takes the Jacobi form, which fits without.
+    const int staged = rb_mode();
+    MgLaunch& M = B.M;
+    MgLists lists;
+    size_t o_part_mg = 0, o_tab_mg = 0, o_vols = 0, o_tiles = 0, o_blocks = 0, o_levels = 0;
+    if (!B.mg_vols.empty()) {
+        const int mg_tiles = mg_tile(B.hmg, B.mg_vols);
+        mg_lists(B.hmg, B.mg_vols, &lists, &M);
+        B.mg_room = nv == 1 ? lists.blocks.size() : mg_list_room(B.hmg, B.mg_vols);   // a batch's tail is listed anew
+        size_t b = align_up(sizeof(MgDesc) * nv, 256);
+        o_part_mg = b;
+        b = align_up(b + sizeof(double) * 2 * (size_t)mg_tiles, 256);
+        o_tab_mg = b;
+        b = align_up(b + sizeof(float) * kTabEntries * nv, 256);
+        o_vols = b;
+        b = align_up(b + sizeof(int) * lists.vols.size(), 256);
+        o_tiles = b;
+        b = align_up(b + sizeof(int2) * lists.tiles.size(), 256);
+        o_blocks = b;
+        b = align_up(b + sizeof(int2) * B.mg_room, 256);
+        o_levels = b;
+        if (staged != 2) b += mg_floats * sizeof(float);
+        B.mg_mem = dalloc(ctx, b);
+        if (!B.mg_mem) {
+            B.mg_vols.clear();
+            M = MgLaunch{};
+            for (VolState<double>& st : B.hst) st.mg = 0;
+        }
+    }
     std::vector<char> h(meta_bytes, 0);
     std::memcpy(h.data() + o_rb, B.hrb.data(), sizeof(RbDesc) * nv);
     std::memcpy(h.data() + o_vol, B.hvol.data(), sizeof(VolDesc) * nv);
@@ -1234,7 +1256,7 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
     RbLaunch& L = B.L;
     L.ntiles = tiles;
     L.nvol = nv;
-    L.staged = rb_mode();
+    L.staged = staged;
     L.fold_alpha = (nv == 1 && tiles <= kRbFoldMaxTiles) ? 1 : 0;
     L.ty = bs.ty;
     L.ahead = bs.ahead;
@@ -1273,29 +1295,20 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
     L.coef0 = B.hcoef[0];
     e = hipMemcpyAsync(m + o_rb, B.hrb.data(), sizeof(RbDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = ft::rb_setup(L, ctx->stream);
-    MgLists lists;
     if (!B.mg_vols.empty()) {
         // the fused Y+Q pass stores no Y: the levels take its place (8 bytes per padded element,
         // at most 2 floats of which they need, see mg_plan)
-        MgLaunch& M = B.M;
-        if (L.staged != 2) B.mg_mem = dalloc(ctx, mg_floats * sizeof(float));
-        float* mem = L.staged == 2 ? (float*)L.y : (float*)B.mg_mem;
-        for (int i : B.mg_vols) B.hmg[i].mem = L.staged == 2 ? mem + 2 * B.hrb[i].off_c : mem + mg_off[i];
+        char* q = (char*)B.mg_mem;
+        for (int i : B.mg_vols)
+            B.hmg[i].mem = staged == 2 ? (float*)L.y + 2 * B.hrb[i].off_c : (float*)(q + o_levels) + mg_off[i];
         M.vol0 = B.hmg[0];
-        mg_lists(B.hmg, B.mg_vols, &lists, &M);
-        const size_t b_vols = align_up(sizeof(int) * lists.vols.size(), 256);
-        const size_t b_tiles = align_up(sizeof(int2) * lists.tiles.size(), 256);
-        B.mg_room = nv == 1 ? lists.blocks.size() : mg_list_room(B.hmg, B.mg_vols);   // a batch's tail is listed anew
-        B.mg_list = dalloc(ctx, b_vols + b_tiles + sizeof(int2) * B.mg_room);
-        if (!mem || !B.mg_list) return FAST_E_OOM;
-        char* q = (char*)B.mg_list;
-        M.vol = (const MgDesc*)(m + o_mg);
-        M.part = (double*)(m + o_mgpart);
-        M.tab = (float*)(m + o_mgtab);
-        M.vols = (const int*)q;
-        M.tiles = (const int2*)(q + b_vols);
-        M.blocks = (const int2*)(q + b_vols + b_tiles);
-        if (e == hipSuccess) e = hipMemcpyAsync(m + o_mg, B.hmg.data(), sizeof(MgDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
+        M.vol = (const MgDesc*)q;
+        M.part = (double*)(q + o_part_mg);
+        M.tab = (float*)(q + o_tab_mg);
+        M.vols = (const int*)(q + o_vols);
+        M.tiles = (const int2*)(q + o_tiles);
+        M.blocks = (const int2*)(q + o_blocks);
+        if (e == hipSuccess) e = hipMemcpyAsync(q, B.hmg.data(), sizeof(MgDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = mg_upload(M, lists, B.mg_room, ctx->stream);
         if (e == hipSuccess) e = ft::mg_setup(L, M, ctx->stream);
     }
