@@ -107,6 +107,7 @@ struct fast_server {
     fast_server_config cfg{};
     int solver = FAST_CG;
     bool rb = true;                           // CG on the red-black Schur complement
+    int staged = 2;                           // form of its Y and Q passes, for as long as the server lives
     fth::RbShape rbs{4, 0, 2};                // red-black rows per tile and prefetch (tz per request)
     std::thread worker;
     std::mutex mu;
@@ -321,7 +322,7 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     RbLaunch& L = s->RL;
     L.ntiles = tiles;
     L.nvol = s->max_active;
-    L.staged = rb_mode();
+    L.staged = s->staged;
     L.fold_alpha = 0;
     L.solo = 0;
     L.ty = s->rbs.ty;
@@ -694,6 +695,7 @@ int fast_server_create(fast_ctx* ctx, const fast_server_config* cfg, fast_server
     if (s->cfg.iters_per_round <= 0) s->cfg.iters_per_round = 8;
     s->solver = s->cfg.use_bicgstab ? FAST_BICGSTAB : FAST_CG;
     s->rb = (s->solver == FAST_CG);
+    s->staged = rb_mode();
     // one launch set serves every live request: the rows per tile and prefetch distance of the
     // 256^3 size class (the middle of the request sizes), tz per request
     s->rbs = rb_shape(ctx, 256, 256, 256);
@@ -717,7 +719,7 @@ int fast_server_create(fast_ctx* ctx, const fast_server_config* cfg, fast_server
         s->d_mg = (MgDesc*)dalloc(ctx, sizeof(MgDesc) * s->max_active);
         s->d_mgtab = (float*)dalloc(ctx, sizeof(float) * kTabEntries * s->max_active);
         mg_ok = s->d_mg && s->d_mgtab;
-        if (rb_mode() == 2) {   // the fused Y+Q pass stores no Y
+        if (s->staged == 2) {   // the fused Y+Q pass stores no Y
             s->mg_base = s->arena_mem ? (float*)rb_f64(s, 0) : nullptr;
         } else {
             s->mg_own = dalloc(ctx, s->S * 2 * sizeof(float));

@@ -1,0 +1,47 @@
+"""The request loop with preconditioned requests: its settings are those of its creation."""
+import pytest
+
+import fast_amd as F
+from fast_amd import tau as T
+
+pytestmark = pytest.mark.gpu
+CG = 1
+SHAPES = [((64, 50, 48), 0), ((48, 50, 64), 4), ((40, 30, 30), 2)]
+
+
+def solo_and_requests():
+    masks = [F.generate_ellipsoids(s, 12.0, 0.35, 0.6, 4 + i) for i, (s, _) in enumerate(SHAPES)]
+    ps = [T.make_params(d, CG, "mixed", 1e-9, 20000) for _, d in SHAPES]
+    c = T.Context(0)
+    try:
+        solo = [c.volume(m).solve(p)[0] for m, p in zip(masks, ps)]
+    finally:
+        c.close()
+    return solo, masks, ps
+
+
+def serve(s, masks, ps):
+    tickets = [s.submit(m, p) for m, p in zip(masks, ps)]
+    got = {}
+    for _ in tickets:
+        t, r, _ = s.wait(60000)
+        got[t] = r
+    return [got[t] for t in tickets]
+
+
+@pytest.mark.parametrize("at_start,later", [("2", "0"), ("0", "2"), ("2", "1")])
+def test_form_of_the_passes_is_that_of_the_servers_creation(monkeypatch, at_start, later):
+    """The preconditioner's levels lie in the Y vector where the passes do not use it, so a change of
+    FAST_TAU_RB_STAGED while a server lives must not bring that vector into use: every result is
+    the solo solve's, bit for bit."""
+    solo, masks, ps = solo_and_requests()
+    monkeypatch.setenv("FAST_TAU_RB_STAGED", at_start)
+    c = T.Context(0)
+    s = T.Server(c, hbm_budget=256 << 20)
+    try:
+        monkeypatch.setenv("FAST_TAU_RB_STAGED", later)
+        for r, q in zip(serve(s, masks, ps), solo):
+            assert r.status == 0 and (r.tau, r.iterations) == (q.tau, q.iterations)
+    finally:
+        s.close()
+        c.close()
