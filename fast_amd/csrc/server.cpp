@@ -157,7 +157,7 @@ struct fast_server {
     double* d_mgpart = nullptr;
     void* d_mglist = nullptr;                 // launch lists
     size_t mgpart_cap = 0, mglist_cap = 0;
-    float* mg_base = nullptr;                 // level storage, 2 floats per arena element
+    float* mg_base = nullptr;                 // level storage, 2 floats per arena element (null: no preconditioner)
     void* mg_own = nullptr;                   // its own plane where the Y vector is in use
     int ntiles = 0;
 };
@@ -221,7 +221,7 @@ VolState<double> fresh_state(const fast_server* s, const Req* r) {
     v.blowup2 = s->ctx->mixed_blowup2;
     MgDesc plan;
     size_t floats = 0;
-    v.mg = s->rb && mg_plan(r->nx, r->ny, r->nz, r->prm.dir / 2, &plan, &floats) ? 1 : 0;
+    v.mg = s->mg_base && mg_plan(r->nx, r->ny, r->nz, r->prm.dir / 2, &plan, &floats) ? 1 : 0;
     v.mg_stall = s->ctx->mg_stall;
     v.eps2 = s->rb ? 2.220446049250313e-16 * 2.220446049250313e-16 : 1.1920928955078125e-07 * 1.1920928955078125e-07;
     return v;
@@ -244,7 +244,7 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
         d.tile_base = tiles;
         if (!r) continue;
         size_t floats = 0;
-        if (mg_plan(r->nx, r->ny, r->nz, r->prm.dir / 2, &s->h_mg[i], &floats)) {
+        if (s->mg_base && mg_plan(r->nx, r->ny, r->nz, r->prm.dir / 2, &s->h_mg[i], &floats)) {
             s->h_mg[i].mem = s->mg_base + 2 * r->off;
             mv.push_back(i);
         }
@@ -713,21 +713,23 @@ int fast_server_create(fast_ctx* ctx, const fast_server_config* cfg, fast_server
     s->d_zero = (unsigned long long*)dalloc(ctx, sizeof(unsigned long long) * s->max_active);
     s->d_tab = (double*)dalloc(ctx, sizeof(double) * 2 * kTabEntries * s->max_active);
     s->d_rb = (RbDesc*)dalloc(ctx, sizeof(RbDesc) * s->max_active);
-    bool mg_ok = true;
-    if (s->rb) {
+    if (s->rb && s->arena_mem) {
         s->h_mg.assign(s->max_active, MgDesc{});
         s->d_mg = (MgDesc*)dalloc(ctx, sizeof(MgDesc) * s->max_active);
         s->d_mgtab = (float*)dalloc(ctx, sizeof(float) * kTabEntries * s->max_active);
-        mg_ok = s->d_mg && s->d_mgtab;
-        if (s->staged == 2) {   // the fused Y+Q pass stores no Y
-            s->mg_base = s->arena_mem ? (float*)rb_f64(s, 0) : nullptr;
-        } else {
-            s->mg_own = dalloc(ctx, s->S * 2 * sizeof(float));
-            s->mg_base = (float*)s->mg_own;
-            mg_ok = mg_ok && s->mg_own;
+        if (s->staged != 2) s->mg_own = dalloc(ctx, s->S * 2 * sizeof(float));
+        s->mg_base = s->staged == 2 ? (float*)rb_f64(s, 0) : (float*)s->mg_own;   // the fused Y+Q pass stores no Y
+        if (!s->d_mg || !s->d_mgtab || !s->mg_base) {   // no room in the budget: the Jacobi form
+            dfree(ctx, s->d_mg);
+            dfree(ctx, s->d_mgtab);
+            dfree(ctx, s->mg_own);
+            s->d_mg = nullptr;
+            s->d_mgtab = nullptr;
+            s->mg_own = nullptr;
+            s->mg_base = nullptr;
         }
     }
-    if (!mg_ok || !s->arena_mem || !s->d_vol || !s->d_coef || !s->d_st || !s->d_zero || !s->d_tab || !s->d_rb ||
+    if (!s->arena_mem || !s->d_vol || !s->d_coef || !s->d_st || !s->d_zero || !s->d_tab || !s->d_rb ||
         hipHostMalloc((void**)&s->h_st, sizeof(VolState<double>) * s->max_active, hipHostMallocDefault) != hipSuccess ||
         hipStreamCreateWithFlags(&s->up, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&s->up_done) != hipSuccess) {
         (void)hipGetLastError();

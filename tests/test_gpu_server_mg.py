@@ -45,3 +45,22 @@ def test_form_of_the_passes_is_that_of_the_servers_creation(monkeypatch, at_star
     finally:
         s.close()
         c.close()
+
+
+def test_server_within_the_budget_of_the_jacobi_form(monkeypatch):
+    """With separate Y and Q passes the levels need a plane of their own (8 bytes an element beside the arena's
+    23 a voxel).  A context with 8 MB beside a 64 MB arena has no room for it: the server opens all the same
+    and serves in the Jacobi form."""
+    solo, masks, ps = solo_and_requests()
+    monkeypatch.setenv("FAST_TAU_RB_STAGED", "0")
+    c = T.Context(0, 72 << 20)
+    try:
+        s = T.Server(c, hbm_budget=64 << 20, max_active=4)
+        try:
+            for r, q in zip(serve(s, masks, ps), solo):
+                assert r.status == 0 and r.true_rel_residual <= 1e-9
+                assert abs(r.tau - q.tau) <= 1e-6 * q.tau
+        finally:
+            s.close()
+    finally:
+        c.close()
