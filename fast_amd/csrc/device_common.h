@@ -411,9 +411,23 @@ __host__ __device__ __forceinline__ void mixed_after_iteration(VolState<A>* s, A
 // count from 0 again (as at Eigen's first restart), so that the cap leaves the Jacobi form what
 // it had without the cycle.
 template <class A>
-__host__ __device__ __forceinline__ void mg_leave(VolState<A>* s) {
+__host__ __device__ __forceinline__ void mg_leave(VolState<A>* s, int why) {
     s->mg = 0;
+    s->mg_left = why;
     s->iter = 0;
+    s->status = ST_FRESH;
+}
+
+// Where the Jacobi form gets nowhere from the x64 that the cycle left, which holds little but the error it
+// is slowest on (it breaks down, meets the iteration cap, or after a breakdown of the cycle takes kMgBrokeStall
+// iterations without a reliable update), it starts from x0, as without the cycle.
+template <class A>
+__host__ __device__ __forceinline__ void mg_forget(VolState<A>* s) {
+    s->mg = 0;
+    s->mg_left = 0;
+    s->iter = 0;
+    s->refinements = 0;   // the update passes take x0
+    s->restarts += 1;
     s->status = ST_FRESH;
 }
 
@@ -422,14 +436,17 @@ __host__ __device__ __forceinline__ void mg_leave(VolState<A>* s) {
 template <class A>
 __host__ __device__ __forceinline__ void cg_breakdown(VolState<A>* s) {
     s->status = ST_FRESH;
-    if (s->mg) mg_leave(s);
+    if (s->mg)
+        mg_leave(s, MG_BROKE);
+    else if (s->mg_left)
+        mg_forget(s);
 }
 
 // r.z of a preconditioned volume's cycle.  It is negative for every r, as D and A are, unless the cycle, in
 // FP32, has overflowed or is not definite here.
 __host__ __device__ __forceinline__ void mg_beta(VolState<double>* s, double rz) {
     if (!(rz < 0.0) || !__builtin_isfinite(rz)) {
-        mg_leave(s);
+        mg_leave(s, MG_BROKE);
         return;
     }
     if (!s->first) s->beta = rz / s->absnew;
@@ -450,8 +467,13 @@ __host__ __device__ __forceinline__ void mixed_cg_after_iteration(VolState<A>* s
         s->status = ST_UPDATE;
         return;
     }
-    if (s->mg && ++s->mg_since >= s->mg_stall) {
-        mg_leave(s);
+    ++s->mg_since;
+    if (s->mg && s->mg_since >= s->mg_stall) {
+        mg_leave(s, MG_STALLED);
+        return;
+    }
+    if (s->mg_left == MG_BROKE && s->mg_since >= kMgBrokeStall) {
+        mg_forget(s);
         return;
     }
     s->first = 0;
@@ -576,7 +598,12 @@ __host__ __device__ void mixres_update(VolState<double>* s, const double* tot) {
     s->discard = 0;
     s->mg_since = 0;
     s->r64sq = tot[0];
-    if (s->b64sq == 0.0 || !(s->r64sq > s->otol * s->otol * s->b64sq) || s->iter >= s->maxiter) {
+    const bool above = s->r64sq > s->otol * s->otol * s->b64sq;
+    if ((s->mg_left && above && s->iter >= s->maxiter) || ((s->mg || s->mg_left) && s->refinements > 1 && s->r64sq != s->r64sq)) {
+        mg_forget(s);
+        return;
+    }
+    if (s->b64sq == 0.0 || !above || s->iter >= s->maxiter) {
         s->status = ST_IDLE;
         return;
     }

@@ -65,7 +65,7 @@ struct VolState {
     int mg;                        // red-black CG: multigrid preconditioner (MgDesc) instead of Jacobi; x then
                                    // takes its step every iteration (xpend 0..1)
     int mg_since, mg_stall;        // its iterations since the last reliable update, and their limit
-    int pad;
+    int mg_left;                   // the Jacobi form started from an x64 of the cycle: MgLeft
 };
 
 // Vectors of one (batched) solve, concatenated over its volumes (element offset VolDesc::off).
@@ -250,11 +250,16 @@ inline int rb_row_pitch(int hx) { return (hx + 2 + 3) & ~3; }
 // FP32; the CG around it keeps its FP64 arithmetic, FP64 residuals and stopping rule.
 // A volume whose residual has not dropped to its next reliable update within kMgStall iterations
 // (seen at solid conductivities of 1e-6 and 95% solid), or has grown 100-fold since the last one, or
-// whose r.z or p.q break down, goes on with the Jacobi form from its x64.
+// whose r.z or p.q break down, goes on with the Jacobi form from its x64, and where that gets nowhere (mg_forget)
+// from x0.
 // The last level has at most 64 cells and is solved with its inverse.  Level l >= 1 holds, per cell, the right-hand side (overwritten by the solution), the black
 // values of the first sweep, the face coefficients towards x+, y+ and z+, and 1 / diagonal, all
 // for -A (positive).  Levels from `bottom` on are solved by one block per volume in LDS.
 constexpr int kMgStall = 128;           // iterations without a reliable update before the Jacobi form takes over
+// After a breakdown of the cycle, iterations without one before it starts from x0: at solid conductivities of 1e-7 to 1e-9
+// it converges from the x64 in 1 to 420 iterations or not at all.
+constexpr int kMgBrokeStall = 1024;
+enum MgLeft : int { MG_STALLED = 1, MG_BROKE = 2 };
 constexpr int kMgLevels = 20;           // levels of the coarsest hierarchy a solver volume can have
 constexpr int kMgArrays = 6;            // g, t, cx, cy, cz, iv
 constexpr int kMgBottomCells = 5120;    // cells of the levels the one-block kernel keeps in LDS

@@ -29,3 +29,20 @@ def test_breakdown_ends_in_a_converged_solve(ctx):
         assert b.status == 0 and (b.tau, b.iterations, b.refinements) == (r.tau, r.iterations, r.refinements)
     for v in vols:
         v.close()
+
+
+def test_a_solve_that_is_stuck_after_the_breakdown_starts_from_x0(ctx):
+    """Volumes on which the Jacobi form converges from x0 (in 2465, 1845 and 1177 iterations) and not from what
+    the cycle left."""
+    restarts = []
+    for shape, solid, seed, d, ds, tol in (((48, 46, 45), 0.75, 6, 2, 1e-8, 1e-9), ((48, 46, 45), 0.75, 7, 2, 1e-8, 1e-9),
+                                           ((80, 60, 40), 0.7, 6, 0, 1e-9, 1e-10)):
+        vol = ctx.volume(F.generate_ellipsoids(shape, 12.0, 0.35, solid, seed))
+        res, _ = vol.solve(T.make_params(d, CG, "mixed", tol, 4000, (1.0, ds)))
+        ref, _ = vol.solve(T.make_params(d, CG, "double", 1e-11, 40000, (1.0, ds)))
+        vol.close()
+        print(shape, seed, res.iterations, res.restarts, res.tau, ref.tau, ref.iterations)
+        assert res.status == 0 and res.true_rel_residual <= tol
+        assert ref.status == 0 and abs(res.tau - ref.tau) <= 1e-5 * ref.tau
+        restarts.append(res.restarts)
+    assert max(restarts) >= 2

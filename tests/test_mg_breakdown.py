@@ -53,10 +53,41 @@ def test_stall_leaves_the_cycle():
 
 
 def test_the_jacobi_form_keeps_its_cap():
-    """A cap of 12 that nine iterations of a failing cycle have used up in part still leaves 12."""
-    out = run(START + 9 * IT + FAILURES["growth"] + START + 12 * [(PQ, -1.0), (END, 0.5)] + START, max_iter=12)
-    assert [o[2] for o in out[-25:-1:2]] == list(range(0, 12)) and out[-1][2] == 12
-    assert out[-4][0] == status("running") and out[-1][0] not in (status("running"), status("fresh"))
+    """A cap of 12 that nine iterations of a failing cycle have used up in part still leaves 12 from the
+    cycle's x64, and after those 12 from x0 (no updates counted); then the volume ends."""
+    jacobi = 12 * [(PQ, -1.0), (END, 0.5)] + START
+    out = run(START + 9 * IT + FAILURES["growth"] + START + jacobi + START + jacobi, max_iter=12)
+    first, second = out[-26 - len(jacobi):-len(jacobi)], out[-len(jacobi) - 1:]
+    assert [o[2] for o in first[:24:2]] == list(range(0, 12)) and first[-2][:3] == (status("fresh"), 0, 0)
+    assert first[-2][3] == 0 and second[0] == (status("running"), 0, 0, 1)
+    assert second[-1][2] == 12 and second[-1][0] not in (status("running"), status("fresh"))
+
+
+@pytest.mark.parametrize("fail", [[(PQ, -1.0), (END, 1.1e4)], [(PQ, 0.0)]], ids=["growth", "alpha"])
+def test_a_second_breakdown_starts_from_x0(fail):
+    """Where the Jacobi form breaks down from the cycle's x64 as well it starts from x0, as a solve without
+    the cycle does; from there on a breakdown is a fresh start that keeps the count."""
+    begin = START + 3 * IT + FAILURES["residual"] + START
+    out = run(begin + 2 * [(PQ, -1.0), (END, 0.5)] + fail + START + [(PQ, -1.0), (END, 0.5)] + fail)
+    again = len(begin) + 4 + len(fail)
+    assert out[again - 1] == (status("fresh"), 0, 0, 0) and out[again] == (status("running"), 0, 0, 1)
+    assert out[-1] == (status("fresh"), 0, len(fail), 1)
+
+
+def test_slow_after_a_breakdown_starts_from_x0():
+    """1024 iterations without a reliable update from the x64 of a cycle that broke down; after one that was
+    only slow the Jacobi form keeps its cap."""
+    slow = [(PQ, -1.0), (END, 0.5)]
+    broke = run(START + 3 * IT + FAILURES["growth"] + START + 1024 * slow, max_iter=5000)
+    assert broke[-3][2] == 1023 and broke[-1] == (status("fresh"), 0, 0, 0)
+    stalled = run(START + 128 * IT + START + 2000 * slow, max_iter=5000)
+    assert stalled[-1][:3] == (status("running"), 0, 2000)
+
+
+def test_a_residual_that_is_not_finite_starts_from_x0():
+    out = run(START + 3 * IT + [(CYCLE, -1.0), (PQ, -1.0), (END, 1e-4), (UPDATE, NAN)] + START)
+    assert out[-2] == (status("fresh"), 0, 0, 0) and out[-1] == (status("running"), 0, 0, 1)
+    assert run([(UPDATE, NAN)])[-1][0] not in (status("running"), status("fresh"))   # the system's own
 
 
 @pytest.mark.parametrize("fail", [[(PQ, -1.0), (END, 1.1e4)], [(PQ, 0.0)]], ids=["growth", "alpha"])
