@@ -667,8 +667,13 @@ void worker_main(fast_server* s) {
             return;
         }
         std::vector<int> fin;
-        for (int i = 0; i < s->max_active; ++i)
-            if (s->slots[i] && s->h_st[i].status == ST_IDLE) fin.push_back(i);
+        bool cycling = false;
+        for (int i = 0; i < s->max_active; ++i) {
+            if (!s->slots[i]) continue;
+            if (s->h_st[i].status == ST_IDLE) fin.push_back(i);
+            cycling = cycling || s->h_st[i].mg;
+        }
+        if (!cycling) s->ML.nvol = 0;   // every live request has left the preconditioner, until the next rebuild
         if (!fin.empty()) {
             int rc = retire(s, fin);
             if (rc == FAST_OK) rc = rebuild(s, {});

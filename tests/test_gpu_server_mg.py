@@ -64,3 +64,19 @@ def test_server_within_the_budget_of_the_jacobi_form(monkeypatch):
             s.close()
     finally:
         c.close()
+
+
+def test_requests_that_leave_the_preconditioner_end_as_alone(monkeypatch):
+    """With a limit of two iterations without a reliable update every request leaves the cycle, and the
+    rounds are the Jacobi form's until one more is admitted: the solo results, bit for bit."""
+    monkeypatch.setenv("FAST_TAU_MG_STALL", "2")
+    solo, masks, ps = solo_and_requests()
+    assert [r.restarts >= 1 for r in solo] == [True, True, False]
+    c = T.Context(0)
+    s = T.Server(c, hbm_budget=256 << 20, max_active=2)   # the third is admitted once another ends
+    try:
+        for r, q in zip(serve(s, masks, ps), solo):
+            assert r.status == 0 and (r.tau, r.iterations, r.restarts) == (q.tau, q.iterations, q.restarts)
+    finally:
+        s.close()
+        c.close()
