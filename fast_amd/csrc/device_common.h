@@ -658,43 +658,6 @@ __device__ __forceinline__ unsigned rb_index(const RbDesc& d, int k, int y, int 
     return (unsigned)(k + 1) + (unsigned)d.px * (unsigned)(y + 1) + d.pp * (unsigned)(z + 1);
 }
 
-// A value that is the same in every lane of the block, kept in scalar registers: after a branch
-// between the kernel's arguments and memory the compiler does not see it by itself, and base
-// pointers in vector registers cost the marches their occupancy.
-template <class T>
-__device__ __forceinline__ T uniform(T v) {
-    static_assert(sizeof(T) % 4 == 0, "32-bit words");
-    union {
-        T t;
-        int w[sizeof(T) / 4];
-    } u{v};
-#pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 4; ++i) u.w[i] = __builtin_amdgcn_readfirstlane(u.w[i]);
-    return u.t;
-}
-
-// Volume, batch tile, descriptor and coefficients of a red-black block.
-__device__ __forceinline__ int rb_vol(const RbLaunch& L, int slot) { return uniform(L.solo ? 0 : L.tile_vol[slot]); }
-__device__ __forceinline__ int rb_tile(const RbLaunch& L, int slot) {
-    return uniform(L.solo || !L.tile_id ? slot : L.tile_id[slot]);
-}
-__device__ __forceinline__ RbDesc rb_desc(const RbLaunch& L, int v) {
-    RbDesc d;
-    if (L.solo)
-        d = L.vol0;
-    else
-        d = L.vol[v];
-    return uniform(d);
-}
-__device__ __forceinline__ Coef<double> rb_coef(const RbLaunch& L, int v) {
-    Coef<double> c;
-    if (L.solo)
-        c = L.coef0;
-    else
-        c = L.coef[v];
-    return uniform(c);
-}
-
 // Compile-time integer, used to unroll a march with constant register indices.
 template <int N>
 struct IC {

@@ -65,24 +65,18 @@ __global__ __launch_bounds__(kRbTX*(TY + 3)) __attribute__((amdgpu_waves_per_eu(
     static_assert(kRbTX == 64 && NPO <= 3 * 64, "one p-only point per lane of waves TY .. TY+2");
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= M.ntiles) return;
-    int2 tl{0, slot};
-    if (!L.solo) tl = M.tiles[slot];
-    const int v = uniform(tl.x), lt = uniform(tl.y);
+    const int2 tl = M.tiles[slot];
+    const int v = tl.x, lt = tl.y;
     const VolState<double>* vs = L.st + v;
     if (vs->status != ST_RUNNING || !vs->mg) return;
-    const RbDesc d = rb_desc(L, v);
-    MgFine md;
-    if (L.solo)
-        md = mg_fine(M.vol0, POST);
-    else
-        md = mg_fine(M.vol[v], POST);
-    md = uniform(md);
+    const RbDesc d = L.vol[v];
+    const MgFine md = mg_fine(M.vol[v], POST);
     __shared__ float tab[kTabEntries];
     __shared__ FacePair<float> ftab[8];
     __shared__ float pbuf[2][PW * PH + 1];
     __shared__ float ybuf[R][YW * YH + 1];
     __shared__ float rows[2][TY / 2][kRbTX];
-    const Coef<double> c = rb_coef(L, v);
+    const Coef<double> c = L.coef[v];
     const Coef<float> cf{(float)c.ci0, (float)c.ci1, (float)c.ci2, (float)c.cb0, (float)c.cb1, 0.0f, 0.0f, 0.0f, 0.0f};
     for (int i = (int)threadIdx.x; i < kTabEntries; i += NT) tab[i] = M.tab[(long long)v * kTabEntries + i];
     if (threadIdx.x < 8) ftab[threadIdx.x] = face_pair(cf, (int)threadIdx.x);
@@ -306,8 +300,6 @@ struct MgLevelArgs {
     const MgDesc* vol;
     const int2* blocks;
     int nblk, lev, tz;
-    float* mem;         // solo launches: the volume's level storage, this level and the next
-    MgLevel la, lc;
 };
 
 struct Float2 {   // two neighbouring floats at any element
@@ -342,20 +334,10 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_level(MgLevelArgs A) {
     __shared__ float rows[2][TY / 2][TK];
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= A.nblk) return;
-    int2 b{0, slot};
-    MgLevel la = A.la, lc = A.lc;
-    float* mem = A.mem;
-    if (!mem) {   // not a solo launch
-        b = A.blocks[slot];
-        la = A.vol[b.x].lev[A.lev];
-        lc = A.vol[b.x].lev[A.lev + 1];
-        mem = A.vol[b.x].mem;
-    }
+    const int2 b = A.blocks[slot];
+    const MgLevel la = A.vol[b.x].lev[A.lev], lc = A.vol[b.x].lev[A.lev + 1];
+    float* mem = A.vol[b.x].mem;
     if (A.st[b.x].status != ST_RUNNING || !A.st[b.x].mg) return;
-    b = uniform(b);
-    la = uniform(la);
-    lc = uniform(lc);
-    mem = uniform(mem);
     const int nx = la.nx, ny = la.ny, nz = la.nz, cx = lc.nx, cy = lc.ny;
     const unsigned nxy = (unsigned)nx * (unsigned)ny, cxy = (unsigned)cx * (unsigned)cy;
     const float* G = mem + la.off;
@@ -512,7 +494,7 @@ __device__ __forceinline__ MgCell lds_cell(const LdsLev& q, unsigned C, int j, i
 __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLaunch M) {
     __shared__ float sm[kMgArrays][kMgBottomCells];
     __shared__ MgLevel sl[kMgLevels];
-    const int v = L.solo ? 0 : M.vols[blockIdx.x];
+    const int v = M.vols[blockIdx.x];
     if (L.st[v].status != ST_RUNNING || !L.st[v].mg) return;
     const MgDesc& d = M.vol[v];
     const int tid = (int)threadIdx.x;
@@ -655,11 +637,10 @@ __global__ __launch_bounds__(kMgBottomThreads) void k_mg_bottom(RbLaunch L, MgLa
 // r.z of one preconditioned volume, then beta = r.z / (previous r.z).  Where mg_beta ends the cycle the passes of
 // this iteration leave the volume alone; x's pending step is in the buffer the cycle did not write.
 __global__ __launch_bounds__(kFinThreads) void k_mg_fin(RbLaunch L, MgLaunch M) {
-    const int v = L.solo ? 0 : M.vols[blockIdx.x];
+    const int v = M.vols[blockIdx.x];
     VolState<double>* s = L.st + v;
     if (s->status != ST_RUNNING || !s->mg) return;
-    const int ntiles = L.solo ? M.vol0.ntiles : M.vol[v].ntiles;
-    const int base = L.solo ? M.vol0.part_base : M.vol[v].part_base;
+    const int ntiles = M.vol[v].ntiles, base = M.vol[v].part_base;
     AccDD sum[1];
     sum[0].init();
     for (int i = (int)threadIdx.x; i < ntiles; i += kFinThreads) {
@@ -1023,8 +1004,7 @@ hipError_t mg_setup(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {
 hipError_t mg_cycle(const RbLaunch& L, const MgLaunch& M, hipStream_t s) {
     const dim3 fb(kRbTX * (kMgTY + 3)), cb(kMgThreads);
     auto args = [&](int l) {
-        return MgLevelArgs{L.st, M.vol, M.blocks + M.blk_off[l], M.nblk[l], l, M.lev_tz[l], L.solo ? M.vol0.mem : nullptr,
-                           M.vol0.lev[l], M.vol0.lev[l + 1]};
+        return MgLevelArgs{L.st, M.vol, M.blocks + M.blk_off[l], M.nblk[l], l, M.lev_tz[l]};
     };
     hipLaunchKernelGGL((k_mg_fine<kMgTY, false>), dim3(M.ntiles), fb, 0, s, L, M);
     for (int l = 0; l < M.nlev; ++l) hipLaunchKernelGGL(k_mg_level<false>, dim3(M.nblk[l]), cb, 0, s, args(l));

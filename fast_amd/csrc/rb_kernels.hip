@@ -111,13 +111,13 @@ template <int KIND, int TY, int AH>
 __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= L.ntiles) return;
-    const int v = rb_vol(L, slot);
-    const int tile = rb_tile(L, slot);   // the tile's index in the batch
-    const RbDesc d = rb_desc(L, v);   // by value: kept in registers across the stores
+    const int v = L.tile_vol[slot];
+    const int tile = L.tile_id ? L.tile_id[slot] : slot;   // the tile's index in the batch
+    const RbDesc d = L.vol[v];   // by value: kept in registers across the stores
     VolState<double>* vs = L.st + v;
     if (vs->status != ST_RUNNING) return;
     __shared__ RbTabs tabs;
-    const Coef<double> c = rb_coef(L, v);
+    const Coef<double> c = L.coef[v];
     rb_load_tables<KIND == RB_Q ? 0 : 1, kRbTX * TY>(L, v, c, tabs);   // Q reads D; P, Y and U read D^-1
     const RbPos ps = rb_pos<TY>(d, tile - d.tile_base);
     constexpr int kColour = (KIND == RB_Y) ? 1 : 0;
@@ -254,14 +254,14 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_q(RbLaunch L) {
     constexpr int RND = (PL + NT - 1) / NT;
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= L.ntiles) return;
-    const int v = rb_vol(L, slot);
-    const int tile = rb_tile(L, slot);   // the tile's index in the batch
-    const RbDesc d = rb_desc(L, v);
+    const int v = L.tile_vol[slot];
+    const int tile = L.tile_id ? L.tile_id[slot] : slot;   // the tile's index in the batch
+    const RbDesc d = L.vol[v];
     const VolState<double>* vs = L.st + v;
     if (vs->status != ST_RUNNING) return;
     __shared__ RbTabs tabs;
     __shared__ U ring[4 * PL];
-    const Coef<double> c = rb_coef(L, v);
+    const Coef<double> c = L.coef[v];
     rb_load_tables<0, NT>(L, v, c, tabs);   // Q reads D only
     const int lt = tile - d.tile_base;
     const int k0 = (lt % d.tiles_x) * kRbTX;
@@ -386,15 +386,15 @@ void k_rb_yq(RbLaunch L) {
     static_assert(kRbTX == 64 && NPO <= 3 * 64, "one p-only point per lane of waves TY .. TY+2");
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= L.ntiles) return;
-    const int v = rb_vol(L, slot);
-    const int tile = rb_tile(L, slot);   // the tile's index in the batch
-    const RbDesc d = rb_desc(L, v);
+    const int v = L.tile_vol[slot];
+    const int tile = L.tile_id ? L.tile_id[slot] : slot;   // the tile's index in the batch
+    const RbDesc d = L.vol[v];
     const VolState<double>* vs = L.st + v;
     if (vs->status != ST_RUNNING) return;
     __shared__ RbTabs tabs;
     __shared__ float pbuf[2][PW * PH + 1];    // + a spare slot for lanes with nothing to store
     __shared__ double ybuf[R][YW * YH + 1];
-    const Coef<double> c = rb_coef(L, v);
+    const Coef<double> c = L.coef[v];
     rb_load_tables<2, NT>(L, v, c, tabs);   // Y reads D_b^-1, Q reads D_r
     const int lt = tile - d.tile_base;
     const int k0 = (lt % d.tiles_x) * kRbTX;
@@ -544,9 +544,9 @@ template <int KIND, int TY>
 __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     if (slot >= L.ntiles) return;
-    const int v = rb_vol(L, slot);
-    const int tile = rb_tile(L, slot);   // the tile's index in the batch
-    const RbDesc d = rb_desc(L, v);
+    const int v = L.tile_vol[slot];
+    const int tile = L.tile_id ? L.tile_id[slot] : slot;   // the tile's index in the batch
+    const RbDesc d = L.vol[v];
     VolState<double>* vs = L.st + v;
     if (KIND == RB_UPD || KIND == RB_Y64 || KIND == RB_R64) {
         const int status = vs->status;
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb(RbLaunch L) {
     }
     constexpr bool kTables = (KIND == RB_Y64 || KIND == RB_R64);
     __shared__ RbTabs tabs;
-    const Coef<double> c = rb_coef(L, v);
+    const Coef<double> c = L.coef[v];
     if (kTables) rb_load_tables<2, kRbTX * TY>(L, v, c, tabs);
     const RbPos ps = rb_pos<TY>(d, tile - d.tile_base);
     constexpr int kColour = (KIND == RB_Y64) ? 1 : 0;

@@ -324,7 +324,6 @@ int rebuild_rb(fast_server* s, const std::vector<Req*>& adm) {
     L.nvol = s->max_active;
     L.staged = s->staged;
     L.fold_alpha = 0;
-    L.solo = 0;
     L.ty = s->rbs.ty;
     L.ahead = s->rbs.ahead;
     L.vol = s->d_rb;

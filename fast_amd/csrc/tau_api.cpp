@@ -1290,9 +1290,6 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         B.hrb[i].code_c[0] = codes + B.hrb[i].off_c;
         B.hrb[i].code_c[1] = codes + total_c + B.hrb[i].off_c;
     }
-    L.solo = nv == 1 ? 1 : 0;
-    L.vol0 = B.hrb[0];
-    L.coef0 = B.hcoef[0];
     e = hipMemcpyAsync(m + o_rb, B.hrb.data(), sizeof(RbDesc) * nv, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = ft::rb_setup(L, ctx->stream);
     if (!B.mg_vols.empty()) {
@@ -1301,7 +1298,6 @@ static int prepare_rb(RbBatch& B, bool use_mg = true) {
         char* q = (char*)B.mg_mem;
         for (int i : B.mg_vols)
             B.hmg[i].mem = staged == 2 ? (float*)L.y + 2 * B.hrb[i].off_c : (float*)(q + o_levels) + mg_off[i];
-        M.vol0 = B.hmg[0];
         M.vol = (const MgDesc*)q;
         M.part = (double*)(q + o_part_mg);
         M.tab = (float*)(q + o_tab_mg);

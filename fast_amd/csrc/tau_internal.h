@@ -201,11 +201,6 @@ struct RbDesc {
 
 struct RbLaunch {
     int ntiles, nvol;
-    int solo;         // 1: a launch over one volume, whose descriptor and coefficients are vol0 and coef0 (a
-                      // kernel's first vector loads then wait for one dependent load, not three) and
-                      // whose tiles are the launch's
-    RbDesc vol0;
-    Coef<double> coef0;
     int ty;           // rows per tile (2, 4, 8, 9, 10, 12 or 13) of every red-black pass of this launch set
     int ahead;        // fused Y+Q pass: planes its loads run ahead (2 or 3)
     int staged;       // 2: Y and Q fused (no Y vector); 1: Q pass with the Y planes staged in LDS; 0: six
@@ -284,7 +279,6 @@ struct MgFine {                         // what the fine-level kernels read of a
     float* g1;
 };
 struct MgLaunch {
-    MgDesc vol0;                        // solo launches (RbLaunch::solo): the volume's descriptor
     int nvol, ntiles;                   // preconditioned volumes, fine tiles
     int nlev, nlev_max;                 // levels launched block-wise; most levels of a volume
     const MgDesc* vol;                  // by volume of the batch
