@@ -34,9 +34,9 @@ __device__ __forceinline__ uint32_t early(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
-// Root of x, pointing every other entry on the way at its grandparent.  An entry only ever moves
-// to a lower ancestor, and one that is not a root never becomes one, so a store
-// that replaces another thread's keeps the entry in its component.
+// Root of x, pointing every other entry on the way at its grandparent.  An entry only ever takes
+// an ancestor of its voxel, and one that is not a root never becomes one, so a store that replaces another
+// thread's, be it with a higher ancestor, keeps the entry in its component.
 __device__ __forceinline__ uint32_t find_halving(uint32_t* P, uint32_t x) {
     for (;;) {
         const uint32_t p = ld(P + x);
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(kScanThreads) void k_assign_roots(const uint32_t* P
 }
 
 // Every other voxel takes its root's label (written by the previous kernel, and not here).  Walking here
-// instead of flattening the entries in a pass of its own: 75 + 29 -> 53 us at 250 x 233 x 241.
+// instead of flattening the entries in a pass of its own: 75 + 29 -> 79 us at 250 x 233 x 241.
 __global__ __launch_bounds__(256) void k_final_labels(const uint32_t* __restrict__ P, long long n, uint32_t* L) {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         uint32_t p = P[i];

@@ -194,7 +194,8 @@ struct AccDD {
 };
 
 // Every solve accumulates its dot products in double-double: a dot then rounds to the same
-// value for any reduction tree, so results do not depend on the tile shape or on the batch.
+// value for any reduction tree unless it lies within about 2^-104 of a rounding tie, so results do not
+// depend on the tile shape or on the batch.
 template <class T, class A>
 struct AccOf {
     using type = AccDD;

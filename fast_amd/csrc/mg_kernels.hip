@@ -5,8 +5,8 @@
 // x1 and leaves the red residual summed over the coarse cells (k_mg_fine<pre>), one adds the
 // prolonged correction while it loads, forms the black values again and writes z with the
 // partial r.z (k_mg_fine<post>).  Slot k of a red row lies in coarse cell k, so restriction and
-// prolongation along x are the identity on the slots.  Coarse levels take four half-sweep
-// kernels each, the levels that fit the LDS of one CU one launch together.
+// prolongation along x are the identity on the slots.  Coarse levels take one launch per half
+// cycle each, the levels that fit the LDS of one CU one launch together.
 #include "device_common.h"
 
 #include <algorithm>
@@ -323,8 +323,8 @@ __device__ __forceinline__ Float2 ld2(const float* p, unsigned i) {
 // its own red cells need are formed again.  Loads take both cells of a pair, two planes ahead.
 // Bound by the chain of steps at 32^3 and 64^3 cells, by loads and memory (five values a cell) beyond.
 // Two launches a half cycle, one per colour with a thread per cell of that colour, took twice the
-// traffic: a cycle's levels of 64^3 (one level) 15.4 -> 9.8 us in half as many launches, of 256^3
-// (three) 75 -> 61 us, of 384^3 (four) 197 -> 151 us, of 24 volumes 100 -> 88 us.  With 4-byte loads
+// traffic: a cycle's levels of 64^3 (one level) 15.4 -> 9.6 us in half as many launches, of 256^3
+// (three) 75 -> 58 us, of 384^3 (four) 197 -> 144 us, of 24 volumes 100 -> 83 us.  With 4-byte loads
 // of the cells' own faces this form took 83 us at 256^3; tiles of 24 rows and 512 threads are even.
 template <bool UP>
 __global__ __launch_bounds__(kMgThreads) void k_mg_level(MgLevelArgs A) {

@@ -208,8 +208,8 @@ __global__ __launch_bounds__(kRbTX* TY) void k_rb_it(RbLaunch L) {
     for (int i = 0; i < AH; ++i) load(ps.z0 + i, in[i]);
     if (KIND == RB_U && L.fold_alpha) {
         // alpha = (r.z) / (p.q) from the Q pass's tile partials of the volume, reduced by every
-        // block alike while its first planes load (a double-double sum rounds to the same value
-        // for any reduction tree), as the finalize would; the block of the volume's first tile
+        // block alike while its first planes load, to what the finalize's sum in another order
+        // rounds to as well (AccOf); the block of the volume's first tile
         // stores it (the finalize after U records it with x's pending step), and a non-finite
         // alpha starts the volume afresh
         __shared__ double pq;

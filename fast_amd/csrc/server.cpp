@@ -788,7 +788,9 @@ int fast_server_submit(fast_server* s, const uint8_t* mask, int nx, int ny, int 
         r->tz = rb_shape(s->ctx, nx, ny, nz).tz;
     } else {
         r->elems = align_up(n, kAlign);
-        // planes per 64 x 8 tile: many requests share a launch, so a volume alone need not fill the chip
+        // planes per 64 x 8 tile: many requests share a launch, so a volume alone need not fill the chip (against one
+        // size class's tuned planes: 12 requests of 64 to 160 edge 373 -> 228 ms, 16 of 32 to 60 22.9 -> 21.1, 3
+        // of 150 to 200 228 -> 218, 4 of 40 to 80 and one of 96 even)
         const long long txy = (long long)((nx + kTX - 1) / kTX) * ((ny + kTY - 1) / kTY);
         r->tz = (int)std::max<long long>(8, std::min<long long>(32, (long long)nz * txy / 1024));
     }

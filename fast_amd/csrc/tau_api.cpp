@@ -176,7 +176,8 @@ static bool shape_compiled(int tx, int ty) {
 // the best 256^3 shape, 64x16x64, is 117 tiles for 256 CUs.  Measured over 14 extents, FP64 and FP32,
 // against sweeps of all shapes: within 3-4% of the best on average and 10% at most, where one
 // shape per power-of-two size class was up to 2.3x off (FP64 CG, an iteration: 160x150x140 148 -> 63
-// us, 191x205x177 168 -> 108, 100^3 53 -> 41, 256^3 243 both).
+// us, 191x205x177 168 -> 108, 100^3 53 -> 41, 256^3 243 both).  The mixed form against those shapes, 16
+// extents from 24x40x33 to 384x320x288: BiCGSTAB 0.97-2.5x, CG on the full grid 0.99-2.5x (256^3 even).
 //
 // Where a batch runs more than two rounds the vectors' traffic counts, which the model does not hold:
 // narrow blocks read more halo, and idle lanes past a row's end cost none.  There the choice is

@@ -236,8 +236,8 @@ inline int rb_row_pitch(int hx) { return (hx + 2 + 3) & ~3; }
 // for the full system A, started from zero with the red residual (the black one is 0):
 //   fine level: Gauss-Seidel red then black, coarse correction, black then red;
 //   coarse levels: cells of 2 x 2 x 2 children (an axis of one cell stays), piecewise constant
-//   transfer, the Galerkin operator's face coefficients (sums of the children's faces) times
-//   1/2, which is the coarse cells' area over their distance; the same sweeps.
+//   transfer, face coefficients of the children's faces in series with half of each side's own, but at
+//   least 0.4 of them (mg_series); the same sweeps.
 // The cycle is symmetric, so CG applies.  On the fine level everything is expressed in
 // x1 = D_r^-1 r: a red sweep from zero gives x1, the black one -Y(x1) = -D_b^-1 A_br x1, the
 // residual left on the red voxels is A_rb Y(x1), and after the correction x2 = x1 + P e the last
@@ -247,9 +247,10 @@ inline int rb_row_pitch(int hx) { return (hx + 2 + 3) & ~3; }
 // (seen at solid conductivities of 1e-6 and 95% solid), or has grown 100-fold since the last one, or
 // whose r.z or p.q break down, goes on with the Jacobi form from its x64, and where that gets nowhere (mg_forget)
 // from x0.
-// The last level has at most 64 cells and is solved with its inverse.  Level l >= 1 holds, per cell, the right-hand side (overwritten by the solution), the black
-// values of the first sweep, the face coefficients towards x+, y+ and z+, and 1 / diagonal, all
-// for -A (positive).  Levels from `bottom` on are solved by one block per volume in LDS.
+// The last level has at most 64 cells and is solved with its inverse.  Level l >= 1 holds, per cell, the
+// right-hand side g, the solution t (during set-up the half-cell faces), the face coefficients towards x+,
+// y+ and z+, and 1 / diagonal, all for -A (positive).  Levels from `bottom` on are solved by one block
+// per volume in LDS.
 constexpr int kMgStall = 128;           // iterations without a reliable update before the Jacobi form takes over
 // After a breakdown of the cycle, iterations without one before it starts from x0: at solid conductivities of 1e-7 to 1e-9
 // it converges from the x64 in 1 to 420 iterations or not at all.
